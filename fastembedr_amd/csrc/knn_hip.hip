@@ -74,24 +74,64 @@ constexpr int kKnnOverRead = knn_tile_pairs(32) * 2 * kKnnThreads + 256;
 
 // ---- 1. prep --------------------------------------------------------------------
 
-// partial[b * d + c] = sum over rows [b * rows_per, (b + 1) * rows_per) of x[., c] in fp64.
+// partial[b * d + c] = sum over rows [b * rows_per, (b + 1) * rows_per) of
+// x[., c] in fp64.  A wave takes 64 columns of every fourth row (row-major:
+// coalesced), the four waves' sums are added in order.  Many short blocks:
+// the sums are chains of dependent loads and adds, and with one chain of 4096
+// rows per column this kernel took 1.1 ms at 70,000 x 50.
 __global__ __launch_bounds__(kPrepThreads) void k_knn_col_partials(const float* __restrict__ x, int n, int d,
                                                                     Strides st, int rows_per,
                                                                     double* __restrict__ partial) {
+  __shared__ double part[kPrepThreads];
   const int r0 = static_cast<int>(blockIdx.x) * rows_per;
   const int r1 = min(n, r0 + rows_per);
-  for (int c = threadIdx.x; c < d; c += kPrepThreads) {
-    double s = 0.0;
-    for (int r = r0; r < r1; ++r) s += static_cast<double>(x[st.at(r, c)]);
-    partial[static_cast<long long>(blockIdx.x) * d + c] = s;
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  constexpr int kWaves = kPrepThreads / kWave;
+  if (st.col_stride == 1) {
+    for (int c0 = 0; c0 < d; c0 += kWave) {
+      const int c = c0 + lane;
+      double s = 0.0;
+      if (c < d) {
+#pragma unroll 8
+        for (int r = r0 + wave; r < r1; r += kWaves) s += static_cast<double>(x[st.at(r, c)]);
+      }
+      part[tid] = s;
+      __syncthreads();
+      if (wave == 0 && c < d) {
+        for (int w = 1; w < kWaves; ++w) s += part[w * kWave + lane];
+        partial[static_cast<long long>(blockIdx.x) * d + c] = s;
+      }
+      __syncthreads();
+    }
+  } else {  // column-major: a wave sums a column's rows, 64 at a time
+    for (int c = wave; c < d; c += kWaves) {
+      double s = 0.0;
+      for (int r = r0 + lane; r < r1; r += kWave) s += static_cast<double>(x[st.at(r, c)]);
+      for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_xor(s, off);
+      if (lane == 0) partial[static_cast<long long>(blockIdx.x) * d + c] = s;
+    }
   }
 }
 
+// Column means from the partials: a block takes 64 columns, its waves every
+// fourth partial.
 __global__ __launch_bounds__(kPrepThreads) void k_knn_col_means(const double* __restrict__ partial, int blocks, int d,
                                                                  int n, double* __restrict__ mean) {
-  for (int c = threadIdx.x; c < d; c += kPrepThreads) {
-    double s = 0.0;
-    for (int b = 0; b < blocks; ++b) s += partial[static_cast<long long>(b) * d + c];
+  __shared__ double part[kPrepThreads];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  constexpr int kWaves = kPrepThreads / kWave;
+  const int c = static_cast<int>(blockIdx.x) * kWave + lane;
+  double s = 0.0;
+  if (c < d) {
+#pragma unroll 8
+    for (int b = wave; b < blocks; b += kWaves) s += partial[static_cast<long long>(b) * d + c];
+  }
+  part[tid] = s;
+  __syncthreads();
+  if (wave == 0 && c < d) {
+    for (int w = 1; w < kWaves; ++w) s += part[w * kWave + lane];
     mean[c] = s / static_cast<double>(n);
   }
 }
@@ -1394,7 +1434,8 @@ int knn_run(const KnnSet& ref, const KnnSet* query, int d, int k, int exclude_se
     idx_out = idx_dev.p;
     dist_out = dist_dev.p;
   }
-  const int rows_per = 4096;
+  // at most 1024 partials a column, of at least 64 rows each
+  const int rows_per = std::max(64, (n + 1023) / 1024);
   const int pblocks = (n + rows_per - 1) / rows_per;
   if ((e = xc.alloc(static_cast<std::size_t>(n_pad) * P + kKnnOverRead)) != hipSuccess ||
       (e = nrm.alloc(n_pad)) != hipSuccess ||
@@ -1417,7 +1458,7 @@ int knn_run(const KnnSet& ref, const KnnSet* query, int d, int k, int exclude_se
   // both sets are centred on the references' column means (and projected
   // on the references' leading directions when wider than kKnnMaxDim)
   k_knn_col_partials<<<pblocks, kPrepThreads, 0, stream>>>(xr, n, d, str, rows_per, partial.p);
-  k_knn_col_means<<<1, kPrepThreads, 0, stream>>>(partial.p, pblocks, d, n, mean.p);
+  k_knn_col_means<<<(d + kWave - 1) / kWave, kPrepThreads, 0, stream>>>(partial.p, pblocks, d, n, mean.p);
   if (project) {
     if ((e = basis.alloc(static_cast<std::size_t>(d) * kProjDim)) != hipSuccess) return fail("hipMalloc(KNN basis)", e);
     if ((e = knn_projection_basis(xr, str, n, d, mean.p, basis.p, stream)) != hipSuccess)
