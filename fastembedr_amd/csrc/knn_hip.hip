@@ -66,8 +66,11 @@ constexpr int kPrepThreads = 256;
 
 // Row pitch of xc for d dimensions: a multiple of 4 plus 2.
 __host__ __device__ constexpr int knn_pitch(int d) { return (d + 3) / 4 * 4 + 2; }
-// float2 copies per thread that stage one 64 x P tile (P <= 4 MAXM + 2).
-__host__ __device__ constexpr int knn_tile_pairs(int maxm) { return (4 * maxm + 2 + 7) / 8; }
+// float2 copies per thread that stage one 64 x P tile of at most nc chunks of
+// 4 dimensions (P <= 4 nc + 2).
+__host__ __device__ constexpr int knn_tile_pairs(int nc) { return (4 * nc + 2 + 7) / 8; }
+// A row's buffer holds this many kp between cuts (and a tile's 64 more).
+constexpr int kKnnBufferRoom = 3;
 // xc is read up to this many floats past its last tile (whole staging copies
 // and the last query row's A loads)
 constexpr int kKnnOverRead = knn_tile_pairs(32) * 2 * kKnnThreads + 256;
@@ -537,59 +540,11 @@ __global__ __launch_bounds__(kKnnRefTile) void k_knn_tile_bounds(const float* __
 }
 
 // ---- sorting inside one wave ------------------------------------------------------
-// PER keys per lane; element E = j * 64 + lane (j = register).  Ascending
-// bitonic sort of the 64 * PER keys.
-
-__device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int mask) {
-  const int lo = __shfl_xor(static_cast<int>(v & 0xffffffffull), mask);
-  const int hi = __shfl_xor(static_cast<int>(v >> 32), mask);
-  return (static_cast<unsigned long long>(static_cast<unsigned int>(hi)) << 32) | static_cast<unsigned int>(lo);
-}
-
-// The stage loops stay rolled (size and distance are wave-uniform); only
-// the per-register work is unrolled, with the in-lane distance a template
-// argument so that registers are never indexed at run time.
-template <int PER, int JD>
-__device__ __forceinline__ void inlane_step_u64(unsigned long long (&key)[PER], int lane, int size) {
-#pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    if ((j & JD) == 0) {
-      const bool asc = ((j * kWave + lane) & size) == 0;
-      const unsigned long long a = key[j], b = key[j | JD];
-      const bool swap = asc ? (a > b) : (a < b);
-      key[j] = swap ? b : a;
-      key[j | JD] = swap ? a : b;
-    }
-  }
-}
-
-template <int PER>
-__device__ __forceinline__ void wave_sort_u64(unsigned long long (&key)[PER], int lane) {
-  constexpr int N = PER * kWave;
-  for (int size = 2; size <= N; size <<= 1) {
-    for (int dist = size >> 1; dist > 0; dist >>= 1) {
-      if (dist >= kWave) {
-        switch (dist / kWave) {
-          case 1: if constexpr (PER > 1) inlane_step_u64<PER, 1>(key, lane, size); break;
-          case 2: if constexpr (PER > 2) inlane_step_u64<PER, 2>(key, lane, size); break;
-          case 4: if constexpr (PER > 4) inlane_step_u64<PER, 4>(key, lane, size); break;
-          case 8: if constexpr (PER > 8) inlane_step_u64<PER, 8>(key, lane, size); break;
-          default: break;
-        }
-      } else {
-        const bool lower = (lane & dist) == 0;
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-          const unsigned long long other = shfl_xor_u64(key[j], dist);
-          const bool keep_min = lower == (((j * kWave + lane) & size) == 0);
-          key[j] = keep_min ? (other < key[j] ? other : key[j]) : (other > key[j] ? other : key[j]);
-        }
-      }
-    }
-  }
-}
-
-// (d2, index) pairs in fp64 / int: same network, lexicographic order.
+// Ascending bitonic sort of 64 * PER (d2, index) pairs, lexicographic; element
+// E = j * 64 + lane (j = register).  The stage loops stay rolled (size and
+// distance are wave-uniform); only the per-register work is unrolled, with the
+// in-lane distance a template argument so that registers are never indexed at
+// run time.
 template <int PER, int JD>
 __device__ __forceinline__ void inlane_step_pairs(double (&d2)[PER], int (&id)[PER], int lane, int size) {
 #pragma unroll
@@ -651,42 +606,68 @@ __device__ __forceinline__ float from_ordered_bits(unsigned int o) {
   return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
 }
 
-__device__ __forceinline__ unsigned long long cand_key(uint2 c) {
-  return (static_cast<unsigned long long>(c.x) << 32) | c.y;
-}
+// Entries a cut may keep beyond kp: the cut's search ends as soon as it
+// leaves kp to kp + kKnnSlack of them.
+constexpr int kKnnSlack = 16;
 
-// Sorts the row's buffer of (ordered s bits, index) entries and keeps its kp
-// best (in order at its front); returns the new count, and the new
-// threshold (the kp-th s) through thr when kp were seen.
-template <int B>
-__device__ __noinline__ int compact_row(uint2* __restrict__ row_buf, int cnt, int kp, int lane, float* thr) {
-  constexpr int PER = B / kWave;
+// Cuts the row's buffer of (ordered s bits, index) entries, cnt > kp of them,
+// to those below a cut value that leaves kp to kp + kKnnSlack (exactly kp of
+// them where more share one value); returns their number and, through thr,
+// the cut: every entry dropped, now or later, has s >= *thr.  Only which
+// entries are below the cut matters, not their order, so the cut is found by
+// bisecting the bits of s with one compare and one popcount per 64 entries
+// and step (10 to 25 steps; lo0: below every s of the row).  A bitonic sort
+// of the same 512 entries issued some 15 times the instructions and, through
+// lane permutes, kept the LDS pipe busy: it took three quarters of the scan.
+template <int PER>
+__device__ __forceinline__ int cut_row(uint2* __restrict__ row_buf, int cnt, int kp, float lo0, int lane,
+                                       float* thr) {
   // The entries were stored by other lanes of this wave: wait until those
   // stores are done (the CU's L1 is shared by the workgroup).
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-  unsigned long long key[PER];
+  uint2 ent[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int e = j * kWave + lane;
-    key[j] = e < cnt ? cand_key(row_buf[e]) : ~0ull;
+    ent[j] = e < cnt ? row_buf[e] : make_uint2(0xffffffffu, 0u);
   }
-  wave_sort_u64<PER>(key, lane);
+  unsigned int lo = ordered_bits(lo0), hi = ordered_bits(*thr);  // fewer than kp below lo, all below hi
+  unsigned int cut = 0u;
+  int below_lo = 0;
+  while (hi - lo > 1u) {
+    const unsigned int mid = lo + (hi - lo) / 2u;
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) c += __popcll(__ballot(ent[j].x < mid));
+    if (c < kp) {
+      lo = mid;
+      below_lo = c;
+    } else if (c > kp + kKnnSlack) {
+      hi = mid;
+    } else {
+      cut = mid;
+      break;
+    }
+  }
+  const bool tied = cut == 0u;  // entries equal to lo make up the kp
+  if (tied) cut = lo;
+  int kept = 0, ties_left = tied ? kp - below_lo : 0;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int e = j * kWave + lane;
-    if (e < kp && e < cnt)
-      row_buf[e] = make_uint2(static_cast<unsigned int>(key[j] >> 32), static_cast<unsigned int>(key[j]));
+    const bool eq = tied && ent[j].x == lo;
+    const unsigned long long me = __ballot(eq);
+    const int eq_rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+        static_cast<unsigned int>(me >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned int>(me), 0u)));
+    const bool keep = ent[j].x < cut || (eq && eq_rank < ties_left);
+    ties_left = max(0, ties_left - static_cast<int>(__popcll(me)));
+    const unsigned long long m = __ballot(keep);
+    const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+        static_cast<unsigned int>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned int>(m), 0u)));
+    if (keep) row_buf[kept + rank] = ent[j];
+    kept += __popcll(m);
   }
-  if (cnt >= kp) {
-    // element kp - 1 sits in lane (kp - 1) % 64, register (kp - 1) / 64
-    unsigned int bits = 0;
-#pragma unroll
-    for (int j = 0; j < PER; ++j)
-      if (j == (kp - 1) / kWave) bits = static_cast<unsigned int>(key[j] >> 32);
-    bits = __shfl(static_cast<int>(bits), (kp - 1) % kWave);
-    *thr = from_ordered_bits(bits);
-  }
-  return min(cnt, kp);
+  *thr = from_ordered_bits(cut);
+  return kept;
 }
 
 // Query list position p -> point index.
@@ -694,73 +675,58 @@ __device__ __forceinline__ int query_id(const int* __restrict__ qlist, int q_off
   return qlist != nullptr ? qlist[p] : q_offset + p;
 }
 
-// Per wave row state in LDS: threshold, count and squared norm of each of its
-// 32 queries.
+// Per wave row state in LDS: squared norm of each of its 32 queries, and
+// thresholds and counts while rows are cut (between cuts they live in
+// registers).
 struct alignas(16) WaveRows {
   float thr[kKnnWaves][kKnnWaveQueries];
   int cnt[kKnnWaves][kKnnWaveQueries];
   float nq[kKnnWaves][kKnnWaveQueries];  // |q|^2
 };
 
-// The dot products of a tile: per chunk m of 4 dimensions, one float2 LDS
-// read of the lane's query (dims 4m + 2h, 4m + 2h + 1) and one per block of
-// 32 references (reference c32, the same dims), then four MFMA steps.  The
-// next chunk's operands are read while the current chunk's steps run (the
-// read one chunk past the last stays inside the LDS rows and is not used);
-// the first chunk starts both accumulators from zero.
-__device__ __forceinline__ void knn_chunk_mfma(float2 a, float2 b0, float2 b1, v16f& acc0, v16f& acc1) {
-  acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b0.x, acc0, 0, 0, 0);
-  acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b1.x, acc1, 0, 0, 0);
-  acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b0.y, acc0, 0, 0, 0);
-  acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b1.y, acc1, 0, 0, 0);
-}
-
-__device__ __forceinline__ void knn_tile_dots(int chunks, const float* qa, const float* col0, const float* col1,
+// The dot products of a tile: NC chunks of 4 dimensions; per chunk the lane
+// holds its query's dims 4m + 2h, 4m + 2h + 1 in registers (zero past the
+// last dimension) and reads one float2 per block of 32 references (reference
+// c32, the same dims), then four MFMA steps.  Reads past a row's end meet the
+// zero query dims; they stay inside the staged copy, whose floats are finite.
+template <int NC>
+__device__ __forceinline__ void knn_tile_dots(const float2 (&qv)[NC], const float* col0, const float* col1,
                                               v16f& acc0, v16f& acc1) {
-  const float2* const q2 = reinterpret_cast<const float2*>(qa);
   const float2* const c0 = reinterpret_cast<const float2*>(col0);
   const float2* const c1 = reinterpret_cast<const float2*>(col1);
-  float2 xa = q2[0], x0 = c0[0], x1 = c1[0];
-  float2 ya = q2[2], y0 = c0[2], y1 = c1[2];
   const v16f zero = {0};
-  acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(xa.x, x0.x, zero, 0, 0, 0);
-  acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(xa.x, x1.x, zero, 0, 0, 0);
-  acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(xa.y, x0.y, acc0, 0, 0, 0);
-  acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(xa.y, x1.y, acc1, 0, 0, 0);
-  for (int m = 1; m < chunks; m += 2) {
-    // chunk m is in y; read chunk m + 1 into x
-    xa = q2[2 * m + 2];
-    x0 = c0[2 * m + 2];
-    x1 = c1[2 * m + 2];
-    knn_chunk_mfma(ya, y0, y1, acc0, acc1);
-    if (m + 1 >= chunks) break;
-    // chunk m + 1 is in x; read chunk m + 2 into y
-    ya = q2[2 * m + 4];
-    y0 = c0[2 * m + 4];
-    y1 = c1[2 * m + 4];
-    knn_chunk_mfma(xa, x0, x1, acc0, acc1);
+  acc0 = zero;
+  acc1 = zero;
+#pragma unroll
+  for (int m = 0; m < NC; ++m) {
+    const float2 b0 = c0[2 * m], b1 = c1[2 * m];
+    acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(qv[m].x, b0.x, acc0, 0, 0, 0);
+    acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(qv[m].x, b1.x, acc1, 0, 0, 0);
+    acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(qv[m].y, b0.y, acc0, 0, 0, 0);
+    acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(qv[m].y, b1.y, acc1, 0, 0, 0);
   }
 }
 
 // One 64-row block's staging copy for one thread: float2 number tid + 256 s
 // (s < pairs = ceil(P / 8)) of the block's contiguous 64 x P rows (the last
 // copy reads past the block's end, into the next rows or the array's tail
-// allowance, and is never used), and one auxiliary float per row: aux0[row]
-// for tid < 64, aux1[row] for 64 <= tid < 128.  Reference tiles carry their
-// norms (aux0); a group's tile centres carry |c|^2 (aux0) and radii (aux1).
-template <int MAXM>
+// allowance, and only zero query dims meet it), and one auxiliary float per
+// row: aux0[row] for tid < 64, aux1[row] for 64 <= tid < 128.  Reference
+// tiles carry their norms (aux0); a group's tile centres carry |c|^2 (aux0)
+// and radii (aux1).
+template <int NC>
 struct TileRegs {
-  float2 v[knn_tile_pairs(MAXM)];
+  float2 v[knn_tile_pairs(NC)];
   float aux;
 };
 
-template <int MAXM>
-__device__ __forceinline__ void knn_load_tile(TileRegs<MAXM>& r, const float* __restrict__ rows,
+template <int NC>
+__device__ __forceinline__ void knn_load_tile(TileRegs<NC>& r, const float* __restrict__ rows,
                                               const float* __restrict__ aux0, const float* __restrict__ aux1, int t,
                                               int P, int pairs, int tid) {
   const float2* const src = reinterpret_cast<const float2*>(rows + static_cast<long long>(t) * kKnnRefTile * P);
 #pragma unroll
-  for (int s = 0; s < knn_tile_pairs(MAXM); ++s)
+  for (int s = 0; s < knn_tile_pairs(NC); ++s)
     if (s < pairs) r.v[s] = src[tid + s * kKnnThreads];
   if (tid < kKnnRefTile)
     r.aux = aux0[t * kKnnRefTile + tid];
@@ -768,38 +734,27 @@ __device__ __forceinline__ void knn_load_tile(TileRegs<MAXM>& r, const float* __
     r.aux = aux1[t * kKnnRefTile + tid - kKnnRefTile];
 }
 
-// LDS of a scan block, in floats: the staged 64 rows (pairs * 512), aux0
-// (64), aux1 (64), then the 128 query rows (pitch P) and 4 floats for the
-// read one chunk past the last row.
+// LDS of one staged block, in floats: the 64 rows (pairs * 512), aux0 (64),
+// aux1 (64).  A scan block holds two, so that one is filled while the other
+// is read and a step needs one barrier.
 __host__ __device__ constexpr int knn_lds_aux(int P) { return (P + 7) / 8 * 2 * kKnnThreads; }
-__host__ __device__ constexpr int knn_lds_queries(int P) { return knn_lds_aux(P) + 2 * kKnnRefTile; }
-__host__ __device__ constexpr int knn_scan_lds_floats(int P) { return knn_lds_queries(P) + kKnnQueryBlock * P + 4; }
+__host__ __device__ constexpr int knn_lds_tile(int P) { return knn_lds_aux(P) + 2 * kKnnRefTile; }
+__host__ __device__ constexpr int knn_scan_lds_floats(int P) { return 2 * knn_lds_tile(P); }
 
-template <int MAXM>
-__device__ __forceinline__ void knn_store_tile(const TileRegs<MAXM>& r, float* dst, int P, int pairs, int tid) {
+template <int NC>
+__device__ __forceinline__ void knn_store_tile(const TileRegs<NC>& r, float* dst, int P, int pairs, int tid) {
   float2* const d2 = reinterpret_cast<float2*>(dst);
 #pragma unroll
-  for (int s = 0; s < knn_tile_pairs(MAXM); ++s)
+  for (int s = 0; s < knn_tile_pairs(NC); ++s)
     if (s < pairs) d2[tid + s * kKnnThreads] = r.v[s];
   if (tid < 2 * kKnnRefTile) dst[knn_lds_aux(P) + tid] = r.aux;
 }
 
-// Lower bound of |q - r|^2 over a ball (centre c, radius rad): (|q - c| -
-// rad)^2 when positive, with |q - c|^2 = |q|^2 + |c|^2 - 2 q.c computed in
-// fp32 and lowered by its rounding bound eps (|q|^2 + |c|^2), the square root
-// and square shaded down by 2^-20.  A ball of radius -inf (padding) bounds
-// at +inf.
-__device__ __forceinline__ float knn_ball_bound(float nq, float nc, float rad, float qc, float eps) {
-  const float d2 = nq + nc - 2.0f * qc - eps * (nq + nc);
-  const float gap = sqrtf(fmaxf(d2, 0.0f)) - rad;
-  return gap > 0.0f ? gap * gap * (1.0f - 0x1.0p-20f) : 0.0f;
-}
-
 // Occupancy: 3 workgroups per CU (3 waves per SIMD) for up to 64 dimensions,
-// 2 above (their LDS, 70 KB at 128 dimensions, allows no more).
-template <int MAXM>
+// 2 above (registers: the queries alone take 2 NC).
+template <int NC>
 constexpr int knn_scan_blocks_per_cu() {
-  return MAXM <= 16 ? 3 : 2;
+  return NC <= 16 ? 3 : 2;
 }
 
 // Reference tiles and their groups: tiles of 64 rows, groups of 64 tiles;
@@ -811,17 +766,21 @@ struct TileGroups {
   const float* radius;  // per tile (-inf past the last tile)
 };
 
-template <int B, int MAXM>
-__global__ __launch_bounds__(kKnnThreads, knn_scan_blocks_per_cu<MAXM>()) void k_knn_scan(
+// PER: registers that hold a row's buffer while it is cut (B <= 64 PER).
+// NC: chunks of 4 dimensions, at least ceil(d / 4).
+// A row's threshold and count are kept in registers, 16 rows per half wave
+// (row 8 (i / 4) + 4 h + i % 4 for accumulator i, the same in the 32 lanes of
+// a half), so that a tile's test and the slots of what it accepts need no
+// LDS; they pass through LDS where rows are cut, about every third tile.
+template <int PER, int NC>
+__global__ __launch_bounds__(kKnnThreads, knn_scan_blocks_per_cu<NC>()) void k_knn_scan(
     const float* __restrict__ xc, const float* __restrict__ nrm, TileGroups tg, const float* __restrict__ xq,
     const float* __restrict__ nrm_q, const int* __restrict__ home, const int* __restrict__ qlist, int q_offset, int nq,
-    int n, int P, int chunks, int kp, float eps_lb, uint2* __restrict__ buf, float* __restrict__ thr_out,
+    int n, int P, int chunks, int kp, int B, float eps_lb, uint2* __restrict__ buf, float* __restrict__ thr_out,
     int* __restrict__ cnt_out, unsigned long long* __restrict__ work) {
   const int pairs = (P + 7) / 8;
   const int aux_at = knn_lds_aux(P);
   extern __shared__ float smem[];
-  float* const rt = smem;                       // the staged rows, then aux0 and aux1
-  float* const qa = smem + knn_lds_queries(P);  // the block's 128 query rows, pitch P
   __shared__ WaveRows rs;
   __shared__ unsigned long long wave_need[kKnnWaves];
   const int tid = static_cast<int>(threadIdx.x);
@@ -831,20 +790,51 @@ __global__ __launch_bounds__(kKnnThreads, knn_scan_blocks_per_cu<MAXM>()) void k
   const int c32 = lane & 31;
   const int p0 = static_cast<int>(blockIdx.x) * kKnnQueryBlock;  // first list position of the block
 
-  // the wave's 32 query rows to LDS (zero rows past the list's end)
+  // the lane's share of query row c32 (zero past the last dimension and past
+  // the list's end)
   const int p_lane = p0 + wave * kKnnWaveQueries + c32;
   const int q_lane = p_lane < nq ? query_id(qlist, q_offset, p_lane) : -1;
-  for (int r = 0; r < kKnnWaveQueries; ++r) {
-    const int q = __shfl(q_lane, r);
-    const float2* const src = reinterpret_cast<const float2*>(xq + static_cast<long long>(q >= 0 ? q : 0) * P);
-    float2* const dst = reinterpret_cast<float2*>(qa + (wave * kKnnWaveQueries + r) * P);
-    for (int e = lane; e < P / 2; e += kWave) dst[e] = q >= 0 ? src[e] : make_float2(0.0f, 0.0f);
+  float2 qv[NC];
+  {
+    const float2* const src = reinterpret_cast<const float2*>(xq + static_cast<long long>(q_lane >= 0 ? q_lane : 0) * P);
+#pragma unroll
+    for (int m = 0; m < NC; ++m)
+      qv[m] = m < chunks && q_lane >= 0 ? src[2 * m + h] : make_float2(0.0f, 0.0f);
   }
   if (lane < kKnnWaveQueries) {
     rs.thr[wave][lane] = q_lane >= 0 ? INFINITY : -INFINITY;  // -inf: no row, accepts nothing
     rs.cnt[wave][lane] = 0;
     rs.nq[wave][lane] = q_lane >= 0 ? nrm_q[q_lane] : 0.0f;
   }
+  float thr[16];
+  int cnt[16];
+  // rows of this lane's half from the wave's LDS copy (written and read by
+  // the same wave: LDS operations of a wave complete in order)
+  auto load_rows = [&]() {
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const float4 t4 = *reinterpret_cast<const float4*>(&rs.thr[wave][8 * g4 + 4 * h]);
+      const int4 c4 = *reinterpret_cast<const int4*>(&rs.cnt[wave][8 * g4 + 4 * h]);
+      thr[4 * g4] = t4.x;
+      thr[4 * g4 + 1] = t4.y;
+      thr[4 * g4 + 2] = t4.z;
+      thr[4 * g4 + 3] = t4.w;
+      cnt[4 * g4] = c4.x;
+      cnt[4 * g4 + 1] = c4.y;
+      cnt[4 * g4 + 2] = c4.z;
+      cnt[4 * g4 + 3] = c4.w;
+    }
+  };
+  auto store_counts = [&]() {
+    if (c32 == 0) {
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        *reinterpret_cast<int4*>(&rs.cnt[wave][8 * g4 + 4 * h]) =
+            make_int4(cnt[4 * g4], cnt[4 * g4 + 1], cnt[4 * g4 + 2], cnt[4 * g4 + 3]);
+    }
+  };
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  load_rows();
 
   // Groups of 64 tiles are visited from the group holding the block's first
   // query's home tile (its own position among the references, or the first
@@ -857,47 +847,69 @@ __global__ __launch_bounds__(kKnnThreads, knn_scan_blocks_per_cu<MAXM>()) void k
   // t + |q|^2 for some query (s = |r|^2 - 2 q.r < t) are staged.  Skipped
   // references count as rejected: their squared distance is at least the
   // query's threshold, as the certificate requires.  The next 64-row block
-  // (tile or group centres) is loaded into registers while one is used.
+  // (tile or group centres) is loaded into registers while one is used, and
+  // stored to the LDS buffer that is not being read: a wave can be one step
+  // ahead of the others at most (the barrier), so the buffer of the step
+  // before is free.
   const int tiles = (n + kKnnRefTile - 1) / kKnnRefTile;
   const int groups = (tiles + kKnnRefTile - 1) / kKnnRefTile;
   const int q_first = query_id(qlist, q_offset, p0);
   const int t0 = __builtin_amdgcn_readfirstlane(home != nullptr ? home[q_first] : q_first / kKnnRefTile);
   const int g0 = t0 / kKnnRefTile;
-  const float* const qrow = qa + (wave * kKnnWaveQueries + c32) * P + 2 * h;
   uint2* const wave_buf = buf + static_cast<long long>(p0 + wave * kKnnWaveQueries) * B;
   unsigned int staged = 0, computed = 0;  // tiles staged by the block, tiles computed by the wave
-  TileRegs<MAXM> pre;
-  knn_load_tile<MAXM>(pre, tg.centre, tg.cnorm, tg.radius, g0, P, pairs, tid);
+  TileRegs<NC> pre;
+  float* rt = smem;
+  float* rt_other = smem + knn_lds_tile(P);
+  knn_load_tile<NC>(pre, tg.centre, tg.cnorm, tg.radius, g0, P, pairs, tid);
   for (int gi = 0; gi < groups; ++gi) {
     const int g = g0 + gi < groups ? g0 + gi : g0 + gi - groups;
-    __syncthreads();  // every wave is done with the rows in LDS
-    knn_store_tile<MAXM>(pre, rt, P, pairs, tid);
+    const int gn = g + 1 < groups ? g + 1 : 0;
+    knn_store_tile<NC>(pre, rt, P, pairs, tid);
     __syncthreads();
+    // most groups need no tile: the next group's centres are on their way
+    if (gi + 1 < groups) knn_load_tile<NC>(pre, tg.centre, tg.cnorm, tg.radius, gn, P, pairs, tid);
     unsigned long long need;  // bit j: tile 64 g + j can hold a candidate of this wave's queries
     {
       v16f acc0, acc1;
-      knn_tile_dots(chunks, qrow, rt + c32 * P + 2 * h, rt + (32 + c32) * P + 2 * h, acc0, acc1);
+      knn_tile_dots<NC>(qv, rt + c32 * P + 2 * h, rt + (32 + c32) * P + 2 * h, acc0, acc1);
       const float nc0 = rt[aux_at + c32], nc1 = rt[aux_at + 32 + c32];
       const float rd0 = rt[aux_at + kKnnRefTile + c32], rd1 = rt[aux_at + kKnnRefTile + 32 + c32];
+      // |q - c| < rad + sqrt(t + |q|^2), squared: |q - c|^2 = |q|^2 + |c|^2 -
+      // 2 q.c in fp32, lowered by its rounding bound eps (|q|^2 + |c|^2), and
+      // the right side raised by 2^-20 for the rounding of the root, the sum
+      // and the square.  A threshold below -|q|^2 (rounding) counts as 0.
       bool need0 = false, need1 = false;
+      const float keep = 1.0f - eps_lb;
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
-        const int row0 = 8 * g4 + 4 * h;
-        const float4 thr4 = *reinterpret_cast<const float4*>(&rs.thr[wave][row0]);
-        const float4 nq4 = *reinterpret_cast<const float4*>(&rs.nq[wave][row0]);
-        const float thr_a[4] = {thr4.x, thr4.y, thr4.z, thr4.w};
+        const float4 nq4 = *reinterpret_cast<const float4*>(&rs.nq[wave][8 * g4 + 4 * h]);
         const float nq_a[4] = {nq4.x, nq4.y, nq4.z, nq4.w};
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const float lim = thr_a[u] + nq_a[u];
-          need0 |= knn_ball_bound(nq_a[u], nc0, rd0, acc0[4 * g4 + u], eps_lb) < lim;
-          need1 |= knn_ball_bound(nq_a[u], nc1, rd1, acc1[4 * g4 + u], eps_lb) < lim;
+          const int i = 4 * g4 + u;
+          const float lim = thr[i] + nq_a[u];
+          const float reach = lim > 0.0f ? __builtin_amdgcn_sqrtf(lim) * (1.0f + 0x1.0p-20f) : 0.0f;
+          const float far0 = fmaxf(rd0 + reach, 0.0f), far1 = fmaxf(rd1 + reach, 0.0f);
+          const float d0 = fmaf(-2.0f, acc0[i], keep * (nq_a[u] + nc0));
+          const float d1 = fmaf(-2.0f, acc1[i], keep * (nq_a[u] + nc1));
+          const bool row = thr[i] > -INFINITY;
+          need0 |= row && d0 < far0 * far0 * (1.0f + 0x1.0p-20f);
+          need1 |= row && d1 < far1 * far1 * (1.0f + 0x1.0p-20f);
         }
       }
       const unsigned long long b0 = __ballot(need0), b1 = __ballot(need1);
       need = ((b0 | (b0 >> 32)) & 0xffffffffull) | (((b1 | (b1 >> 32)) & 0xffffffffull) << 32);
+      // the last group's tiles end with the references
+      const int real = tiles - g * kKnnRefTile;
+      if (real < kKnnRefTile) need &= (1ull << real) - 1ull;
     }
     if (lane == 0) wave_need[wave] = need;
+    {
+      float* const t = rt;
+      rt = rt_other;
+      rt_other = t;
+    }
     __syncthreads();
     // Tiles are taken in order from `rot` (the block's own tile in the first
     // group, so that the thresholds start from the nearest references), as
@@ -910,95 +922,90 @@ __global__ __launch_bounds__(kKnnThreads, knn_scan_blocks_per_cu<MAXM>()) void k
     if (todo != 0ull) {
       cur = __ffsll(static_cast<long long>(todo)) - 1;
       todo &= todo - 1ull;
-      knn_load_tile<MAXM>(pre, xc, nrm, nullptr, g * kKnnRefTile + ((cur + rot) & (kKnnRefTile - 1)), P, pairs,
-                          tid);
-    } else if (gi + 1 < groups) {
-      const int gn = g + 1 < groups ? g + 1 : 0;
-      knn_load_tile<MAXM>(pre, tg.centre, tg.cnorm, tg.radius, gn, P, pairs, tid);
+      knn_load_tile<NC>(pre, xc, nrm, nullptr, g * kKnnRefTile + ((cur + rot) & (kKnnRefTile - 1)), P, pairs, tid);
     }
     while (cur >= 0) {
-      __syncthreads();  // every wave is done with the rows in LDS
-      knn_store_tile<MAXM>(pre, rt, P, pairs, tid);
+      knn_store_tile<NC>(pre, rt, P, pairs, tid);
       __syncthreads();
       int next = -1;
       if (todo != 0ull) {
         next = __ffsll(static_cast<long long>(todo)) - 1;
         todo &= todo - 1ull;
-        knn_load_tile<MAXM>(pre, xc, nrm, nullptr, g * kKnnRefTile + ((next + rot) & (kKnnRefTile - 1)), P, pairs,
-                            tid);
+        knn_load_tile<NC>(pre, xc, nrm, nullptr, g * kKnnRefTile + ((next + rot) & (kKnnRefTile - 1)), P, pairs,
+                          tid);
       } else if (gi + 1 < groups) {
-        const int gn = g + 1 < groups ? g + 1 : 0;
-        knn_load_tile<MAXM>(pre, tg.centre, tg.cnorm, tg.radius, gn, P, pairs, tid);
+        knn_load_tile<NC>(pre, tg.centre, tg.cnorm, tg.radius, gn, P, pairs, tid);
       }
       ++staged;
       if ((need >> cur) & 1ull) {
         ++computed;
         v16f acc0, acc1;
-        knn_tile_dots(chunks, qrow, rt + c32 * P + 2 * h, rt + (32 + c32) * P + 2 * h, acc0, acc1);
+        knn_tile_dots<NC>(qv, rt + c32 * P + 2 * h, rt + (32 + c32) * P + 2 * h, acc0, acc1);
         // filter: s = |r|^2 - 2 q.r below the row's threshold goes to the
-        // row's buffer.  Output i of this lane is row 8 (i / 4) + 4 h + i % 4
-        // of the wave's 32, reference c32 of the 32-reference block.
+        // row's buffer
         const float nr0 = rt[aux_at + c32];
         const float nr1 = rt[aux_at + 32 + c32];
         const unsigned int col0 =
             static_cast<unsigned int>((g * kKnnRefTile + ((cur + rot) & (kKnnRefTile - 1))) * kKnnRefTile + c32);
+        int most = 0;
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int row0 = 8 * g4 + 4 * h;
-          const float4 thr4 = *reinterpret_cast<const float4*>(&rs.thr[wave][row0]);
-          const float thr_a[4] = {thr4.x, thr4.y, thr4.z, thr4.w};
-          float sv[8];
-          unsigned long long m[8];
-          unsigned long long any = 0ull;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            sv[2 * u] = fmaf(-2.0f, acc0[4 * g4 + u], nr0);
-            sv[2 * u + 1] = fmaf(-2.0f, acc1[4 * g4 + u], nr1);
-            m[2 * u] = __ballot(sv[2 * u] < thr_a[u]);
-            m[2 * u + 1] = __ballot(sv[2 * u + 1] < thr_a[u]);
-            any |= m[2 * u] | m[2 * u + 1];
+        for (int i = 0; i < 16; ++i) {
+          const float s0 = fmaf(-2.0f, acc0[i], nr0), s1 = fmaf(-2.0f, acc1[i], nr1);
+          const unsigned long long m0 = __ballot(s0 < thr[i]), m1 = __ballot(s1 < thr[i]);
+          if ((m0 | m1) != 0ull) {
+            // slots of the lane's half: block 0's references, then block 1's
+            const unsigned int l0 = static_cast<unsigned int>(m0), u0 = static_cast<unsigned int>(m0 >> 32);
+            const unsigned int l1 = static_cast<unsigned int>(m1), u1 = static_cast<unsigned int>(m1 >> 32);
+            const int pre0 = h ? __builtin_amdgcn_mbcnt_hi(u0, 0u) : __builtin_amdgcn_mbcnt_lo(l0, 0u);
+            const int pre1 = h ? __builtin_amdgcn_mbcnt_hi(u1, 0u) : __builtin_amdgcn_mbcnt_lo(l1, 0u);
+            const int n0 = h ? __popc(u0) : __popc(l0);
+            const int n1 = h ? __popc(u1) : __popc(l1);
+            uint2* const row = wave_buf + (8 * (i / 4) + 4 * h + i % 4) * B + cnt[i];
+            if (s0 < thr[i]) row[pre0] = make_uint2(ordered_bits(s0), col0);
+            if (s1 < thr[i]) row[n0 + pre1] = make_uint2(ordered_bits(s1), col0 + 32u);
+            cnt[i] += n0 + n1;
           }
-          if (any != 0ull) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              if (m[j] != 0ull) {
-                const int row = row0 + j / 2;
-                const unsigned int half =
-                    h ? static_cast<unsigned int>(m[j] >> 32) : static_cast<unsigned int>(m[j]);
-                const int base = rs.cnt[wave][row];
-                if (sv[j] < thr_a[j / 2])
-                  wave_buf[static_cast<long long>(row) * B + base + __popc(half & ((1u << c32) - 1u))] =
-                      make_uint2(ordered_bits(sv[j]), col0 + (j & 1) * 32u);
-                if (c32 == 0) rs.cnt[wave][row] = base + __popc(half);
-              }
+          most = max(most, cnt[i]);
+        }
+        // rows that could overflow in the next tile are cut to kp (and a few)
+        if (__ballot(most > B - kKnnRefTile) != 0ull) {
+          store_counts();
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+          unsigned long long full = __ballot(lane < kKnnWaveQueries && rs.cnt[wave][c32] > B - kKnnRefTile);
+          while (full != 0ull) {
+            const int r = __ffsll(static_cast<long long>(full)) - 1;
+            full &= full - 1ull;
+            float t = rs.thr[wave][r];
+            const int c = cut_row<PER>(wave_buf + r * B, rs.cnt[wave][r], kp, fmaf(-2.0f, rs.nq[wave][r], -1.0f),
+                                       lane, &t);
+            if (lane == 0) {
+              rs.cnt[wave][r] = c;
+              rs.thr[wave][r] = t;
             }
           }
-        }
-        // rows that could overflow in the next tile: sort, keep kp
-        unsigned long long full = __ballot(lane < kKnnWaveQueries && rs.cnt[wave][c32] > B - kKnnRefTile);
-        while (full != 0ull) {
-          const int r = __ffsll(static_cast<long long>(full)) - 1;
-          full &= full - 1ull;
-          float thr = rs.thr[wave][r];
-          const int c = compact_row<B>(wave_buf + static_cast<long long>(r) * B, rs.cnt[wave][r], kp, lane, &thr);
-          if (lane == 0) {
-            rs.cnt[wave][r] = c;
-            rs.thr[wave][r] = thr;
-          }
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+          load_rows();
         }
       }
       cur = next;
+      float* const t = rt;
+      rt = rt_other;
+      rt_other = t;
     }
   }
-  // final: keep kp per row; the threshold is what a rejected reference beat
+  // final: kp (and a few) per row; the threshold is what a rejected reference
+  // is at or above
+  store_counts();
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   for (int r = 0; r < kKnnWaveQueries; ++r) {
     const int p = p0 + wave * kKnnWaveQueries + r;
     if (p >= nq) break;  // wave-uniform
-    float thr = rs.thr[wave][r];
-    int c = rs.cnt[wave][r];
-    if (c > kp) c = compact_row<B>(wave_buf + static_cast<long long>(r) * B, c, kp, lane, &thr);
+    float t = rs.thr[wave][r];
+    int c = __builtin_amdgcn_readfirstlane(rs.cnt[wave][r]);
+    if (c > kp + kKnnSlack)
+      c = cut_row<PER>(wave_buf + r * B, c, kp, fmaf(-2.0f, rs.nq[wave][r], -1.0f), lane, &t);
     if (lane == 0) {
-      thr_out[p] = thr;
+      thr_out[p] = t;
       cnt_out[p] = c;
     }
   }
@@ -1010,6 +1017,53 @@ __global__ __launch_bounds__(kKnnThreads, knn_scan_blocks_per_cu<MAXM>()) void k
 
 // ---- 3. finalize -------------------------------------------------------------------
 
+// V consecutive floats of a row-major row (aligned to 4 V bytes), as doubles.
+template <int V>
+__device__ __forceinline__ void load_wide(const float* p, double (&out)[V]) {
+  if constexpr (V == 4) {
+    const float4 v = *reinterpret_cast<const float4*>(p);
+    out[0] = v.x;
+    out[1] = v.y;
+    out[2] = v.z;
+    out[3] = v.w;
+  } else if constexpr (V == 2) {
+    const float2 v = *reinterpret_cast<const float2*>(p);
+    out[0] = v.x;
+    out[1] = v.y;
+  } else {
+    out[0] = p[0];
+  }
+}
+
+// Squared distance of row r to the query row, fp64, dimensions in order (the
+// same value for any V).  V > 0: rows are contiguous and d is a multiple of V.
+template <int V>
+__device__ __forceinline__ double knn_sq_dist(const float* __restrict__ xq_in, long long q_at, int q_step,
+                                              const float* __restrict__ xr_in, Strides str, int r, int d) {
+  double s = 0.0;
+  if constexpr (V == 0) {
+    for (int t = 0; t < d; ++t) {
+      const double diff = static_cast<double>(xq_in[q_at + static_cast<long long>(t) * q_step]) -
+                          static_cast<double>(xr_in[str.at(r, t)]);
+      s = fma(diff, diff, s);
+    }
+  } else {
+    const float* const row = xr_in + static_cast<long long>(r) * d;
+    const float* const qrow = xq_in + q_at;
+#pragma unroll 4
+    for (int t = 0; t < d; t += V) {
+      double v[V];
+      load_wide<V>(row + t, v);
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        const double diff = static_cast<double>(qrow[t + u]) - v[u];
+        s = fma(diff, diff, s);
+      }
+    }
+  }
+  return s;
+}
+
 // One wave per query: exact squared distances of the candidates from the
 // input rows (fp64); the query itself is dropped when exclude_self; the rest
 // are sorted by (d2, index) and the first k written as 1-based indices and
@@ -1018,17 +1072,23 @@ __global__ __launch_bounds__(kKnnThreads, knn_scan_blocks_per_cu<MAXM>()) void k
 // rows, identity when null); candidates are reference positions in scan
 // order (rperm maps them to reference input rows).  Uncertified queries are
 // appended to retry.
-template <int B>
+//
+// Bound by the candidates' scattered rows: a lane walks its own row, so a
+// load touches 64 cache lines and the lines a wave has open exceed its share
+// of the L1.  V floats per load (the widest the rows' alignment allows) use
+// more of a line each time it is there, and the query's row, the same for
+// the whole wave, comes through scalar loads.
+template <int PER, int V>
 __global__ __launch_bounds__(kKnnThreads) void k_knn_finalize(
     const float* __restrict__ xq_in, Strides stq, const float* __restrict__ xr_in, Strides str, int n_out, int d,
     const int* __restrict__ qperm, const int* __restrict__ rperm, const int* __restrict__ qlist, int q_offset,
-    int nq, const uint2* __restrict__ buf, const float* __restrict__ thr_in, const int* __restrict__ cnt_in,
+    int nq, int B, const uint2* __restrict__ buf, const float* __restrict__ thr_in, const int* __restrict__ cnt_in,
     const float* __restrict__ nrm_q, const unsigned int* __restrict__ nrm_max_bits, float eps_unit, int k,
     int exclude_self, int half_squared, int* __restrict__ idx_out, float* __restrict__ dist_out,
     int* __restrict__ retry, int* __restrict__ retry_count, int* __restrict__ short_rows) {
-  constexpr int PER = B / kWave;
   const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
-  const int p = static_cast<int>(blockIdx.x) * kKnnWaves + static_cast<int>(threadIdx.x) / kWave;
+  const int p = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * kKnnWaves +
+                                               static_cast<int>(threadIdx.x) / kWave);
   if (p >= nq) return;  // whole wave
   const int qid = query_id(qlist, q_offset, p);
   const int q = qperm != nullptr ? qperm[qid] : qid;
@@ -1047,12 +1107,7 @@ __global__ __launch_bounds__(kKnnThreads) void k_knn_finalize(
       if (exclude_self && r == q) {
         self_here = true;  // sorts last
       } else {
-        double s = 0.0;
-        for (int t = 0; t < d; ++t) {
-          const double diff = static_cast<double>(xq_in[stq.at(q, t)]) - static_cast<double>(xr_in[str.at(r, t)]);
-          s = fma(diff, diff, s);
-        }
-        dd[j] = s;
+        dd[j] = knn_sq_dist<V>(xq_in, stq.at(q, 0), static_cast<int>(stq.at(0, 1)), xr_in, str, r, d);
         id[j] = r;
       }
     }
@@ -1212,62 +1267,100 @@ struct KnnPass {
   unsigned long long* work;  // [0] tiles staged (per block), [1] tiles computed (per wave)
 };
 
-template <int B, int MAXM>
-hipError_t launch_scan(const KnnPass& a, int kp, const int* qlist, int q_offset, int nq, hipStream_t stream) {
+// Candidate buffer entries of a row: room for about 2 kp new ones between
+// cuts (a cut every 2 kp acceptances; a tile's 64 more may arrive before it).
+int buffer_for(int kp) {
+  const int room = (kKnnBufferRoom * kp + kKnnSlack + kWave - 1) / kWave * kWave;
+  return std::min(1024, std::max(128, room + kKnnRefTile));
+}
+
+template <int PER, int NC>
+hipError_t launch_scan(const KnnPass& a, int kp, int B, const int* qlist, int q_offset, int nq, hipStream_t stream) {
   const std::size_t lds = static_cast<std::size_t>(knn_scan_lds_floats(a.P)) * sizeof(float);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_knn_scan<B, MAXM>),
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_knn_scan<PER, NC>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   if (e != hipSuccess) return e;
   const int blocks = (nq + kKnnQueryBlock - 1) / kKnnQueryBlock;
   const float eps_lb = static_cast<float>(4 * a.chunks + 8) * 0x1.0p-23f;
-  k_knn_scan<B, MAXM><<<blocks, kKnnThreads, lds, stream>>>(a.xr, a.nrm_r, a.tg, a.xq, a.nrm_q, a.home, qlist,
-                                                            q_offset, nq, a.n_scan, a.P, a.chunks, kp, eps_lb, a.buf,
-                                                            a.thr, a.cnt, a.work);
+  k_knn_scan<PER, NC><<<blocks, kKnnThreads, lds, stream>>>(a.xr, a.nrm_r, a.tg, a.xq, a.nrm_q, a.home, qlist,
+                                                            q_offset, nq, a.n_scan, a.P, a.chunks, kp, B, eps_lb,
+                                                            a.buf, a.thr, a.cnt, a.work);
   return hipGetLastError();
 }
 
-template <int B>
-hipError_t launch_scan_finalize(const KnnPass& a, int kp, const int* qlist, int q_offset, int nq,
-                                hipStream_t stream) {
+// The scan with the fewest chunks of 4 dimensions that hold the rows (its
+// loops over them are unrolled; the steps past the last dimension are work
+// for nothing, at most a third of them).
+template <int PER>
+hipError_t launch_scan_chunks(const KnnPass& a, int kp, int B, const int* qlist, int q_offset, int nq,
+                              hipStream_t stream) {
   static_assert(kKnnMaxDim <= 4 * 32, "at most 32 chunks of 4 dimensions");
-  hipError_t e = a.chunks <= 16 ? launch_scan<B, 16>(a, kp, qlist, q_offset, nq, stream)
-                                : launch_scan<B, 32>(a, kp, qlist, q_offset, nq, stream);
-  if (e != hipSuccess) return e;
+  if (a.chunks <= 4) return launch_scan<PER, 4>(a, kp, B, qlist, q_offset, nq, stream);
+  if (a.chunks <= 8) return launch_scan<PER, 8>(a, kp, B, qlist, q_offset, nq, stream);
+  if (a.chunks <= 13) return launch_scan<PER, 13>(a, kp, B, qlist, q_offset, nq, stream);
+  if (a.chunks <= 16) return launch_scan<PER, 16>(a, kp, B, qlist, q_offset, nq, stream);
+  if (a.chunks <= 24) return launch_scan<PER, 24>(a, kp, B, qlist, q_offset, nq, stream);
+  return launch_scan<PER, 32>(a, kp, B, qlist, q_offset, nq, stream);
+}
+
+template <int PER, int V>
+hipError_t launch_finalize(const KnnPass& a, int B, const int* qlist, int q_offset, int nq, hipStream_t stream) {
   const float eps_unit = static_cast<float>(4 * a.chunks + 12 + a.proj_slack) * 0x1.0p-23f;
-  k_knn_finalize<B><<<(nq + kKnnWaves - 1) / kKnnWaves, kKnnThreads, 0, stream>>>(
-      a.xq_in, a.stq, a.xr_in, a.str, a.n_out, a.d, a.qperm, a.rperm, qlist, q_offset, nq, a.buf, a.thr, a.cnt,
+  k_knn_finalize<PER, V><<<(nq + kKnnWaves - 1) / kKnnWaves, kKnnThreads, 0, stream>>>(
+      a.xq_in, a.stq, a.xr_in, a.str, a.n_out, a.d, a.qperm, a.rperm, qlist, q_offset, nq, B, a.buf, a.thr, a.cnt,
       a.nrm_q, a.nrm_max_bits, eps_unit, a.k, a.exclude_self, a.half_squared, a.idx_out, a.dist_out, a.retry,
-      a.retry_count,
-      a.short_rows);
+      a.retry_count, a.short_rows);
   return hipGetLastError();
 }
 
-// Candidates per query: k plus a margin of max(32, k / 2) (plus the query
-// itself, which the scan does not skip) on the first pass, doubled for every
-// rerun, at most kKnnMaxCand.
-constexpr int kKnnMaxCand = 1024 - 2 * kKnnRefTile;  // 896
+// The widest load that keeps every row's pieces aligned: rows contiguous in
+// both sets, d a multiple of it and both matrices aligned to it.
+template <int PER>
+hipError_t launch_finalize_width(const KnnPass& a, int B, const int* qlist, int q_offset, int nq,
+                                 hipStream_t stream) {
+  const bool rows = a.stq.at(0, 1) == 1 && a.stq.at(1, 0) == a.d && a.str.at(0, 1) == 1 && a.str.at(1, 0) == a.d;
+  const std::uintptr_t at = reinterpret_cast<std::uintptr_t>(a.xr_in);
+  if (rows && a.d % 4 == 0 && at % 16 == 0) return launch_finalize<PER, 4>(a, B, qlist, q_offset, nq, stream);
+  if (rows && a.d % 2 == 0 && at % 8 == 0) return launch_finalize<PER, 2>(a, B, qlist, q_offset, nq, stream);
+  if (rows) return launch_finalize<PER, 1>(a, B, qlist, q_offset, nq, stream);
+  return launch_finalize<PER, 0>(a, B, qlist, q_offset, nq, stream);
+}
 
-// Smallest buffer with room for kp entries plus at least kp new ones (and a
-// tile's 64) between compactions; 1024 for the largest kp.
-int buffer_for(int kp) {
-  for (int B = 128; B <= 1024; B <<= 1)
-    if (B - kKnnRefTile >= 2 * kp) return B;
-  return 1024;
+// Most candidates per query (kp), so that a cut leaves a buffer of 1024 room
+// for the next tile's.
+constexpr int kKnnMaxCand = 1024 - 2 * kKnnRefTile;  // 896
+static_assert(kKnnMaxCand + kKnnSlack + kKnnRefTile <= 1024, "a cut row takes a whole tile more");
+
+// Candidates per query of the first pass: k (and the query itself, which the
+// scan does not skip) plus a margin, so that few rows miss the certificate;
+// every rerun doubles them.  The finalize sorts a power of two of them, so
+// the margin takes what is left of the one that holds k + k / 5 (at least
+// k + 16), at most k / 2 (at least 32): the certificate needs only the gap
+// of a few neighbours (at 1M x 50, k = 90 its width, eps, is 0.4 neighbour
+// spacings), and both the scan's acceptances and the finalize grow with kp.
+// Projected rows: the bound is looser by the spread outside the projection,
+// so they start with twice the largest margin.
+int first_candidates(int k, bool self, bool project) {
+  const int need = k + (self ? 1 : 0);
+  const int most = need + (project ? 2 : 1) * std::max(32, k / 2);
+  if (project) return std::min(kKnnMaxCand, most);
+  int cap = kWave;
+  while (cap < need + std::max(16, k / 5) + kKnnSlack) cap <<= 1;
+  return std::min(kKnnMaxCand, std::min(cap - kKnnSlack, most));
 }
 
 hipError_t launch_pass(const KnnPass& a, int kp, const int* qlist, int q_offset, int nq, hipStream_t stream) {
-#define FEHIP_KNN_PASS(B_) \
-  case B_:                 \
-    return launch_scan_finalize<B_>(a, kp, qlist, q_offset, nq, stream);
-  switch (buffer_for(kp)) {
-    FEHIP_KNN_PASS(128)
-    FEHIP_KNN_PASS(256)
-    FEHIP_KNN_PASS(512)
-    FEHIP_KNN_PASS(1024)
-    default:
-      return hipErrorInvalidValue;
-  }
-#undef FEHIP_KNN_PASS
+  const int B = buffer_for(kp);
+  hipError_t e = B <= 256   ? launch_scan_chunks<4>(a, kp, B, qlist, q_offset, nq, stream)
+                 : B <= 512 ? launch_scan_chunks<8>(a, kp, B, qlist, q_offset, nq, stream)
+                            : launch_scan_chunks<16>(a, kp, B, qlist, q_offset, nq, stream);
+  if (e != hipSuccess) return e;
+  const int most = kp + kKnnSlack;  // candidates a row can bring
+  if (most <= 64) return launch_finalize_width<1>(a, B, qlist, q_offset, nq, stream);
+  if (most <= 128) return launch_finalize_width<2>(a, B, qlist, q_offset, nq, stream);
+  if (most <= 256) return launch_finalize_width<4>(a, B, qlist, q_offset, nq, stream);
+  if (most <= 512) return launch_finalize_width<8>(a, B, qlist, q_offset, nq, stream);
+  return launch_finalize_width<16>(a, B, qlist, q_offset, nq, stream);
 }
 
 template <typename T>
@@ -1575,13 +1668,15 @@ int knn_run(const KnnSet& ref, const KnnSet* query, int d, int k, int exclude_se
   // kKnnCandEntries in all; a pass launches as many queries at once as they
   // allow (one launch for the whole input up to millions of rows, so that
   // the grid is many rounds of workgroups deep).
-  // (projected rows: the bound is looser by the spread outside the
-  // projection, so the first pass starts with twice the margin)
-  int kp = std::min(kKnnMaxCand, k + (project ? 2 : 1) * std::max(32, k / 2) + (self ? 1 : 0));
+  int kp = first_candidates(k, self, project);
   const std::size_t entries = std::min<std::size_t>(
       kKnnCandEntries, static_cast<std::size_t>(n_out) * static_cast<std::size_t>(buffer_for(kp)));
-  auto batch_for = [&](int kp_) {
-    return static_cast<int>(std::min<std::size_t>(static_cast<std::size_t>(n_out), entries / buffer_for(kp_)));
+  // (batches of equal size: the last rounds of a launch leave CUs idle)
+  auto batch_for = [&](int kp_, int rows) {
+    const int most = static_cast<int>(std::min<std::size_t>(static_cast<std::size_t>(n_out), entries / buffer_for(kp_)));
+    const int launches = (rows + most - 1) / most;
+    const int even = (rows + launches - 1) / launches;
+    return std::min(most, (even + kKnnQueryBlock - 1) / kKnnQueryBlock * kKnnQueryBlock);
   };
   DevBuf<uint2> buf;
   DevBuf<float> thr;
@@ -1626,7 +1721,7 @@ int knn_run(const KnnSet& ref, const KnnSet* query, int d, int k, int exclude_se
   pass.short_rows = counters.p + 1;
   pass.work = work.p;
   const int* main_list = self ? qpos.p : qorder.p;
-  for (int q0 = 0, batch = batch_for(kp); q0 < n_out; q0 += batch) {
+  for (int q0 = 0, batch = batch_for(kp, n_out); q0 < n_out; q0 += batch) {
     const int nq = std::min(batch, n_out - q0);
     if ((e = launch_pass(pass, kp, main_list + q0, 0, nq, stream)) != hipSuccess) return fail("KNN scan launch", e);
   }
@@ -1680,7 +1775,7 @@ int knn_run(const KnnSet& ref, const KnnSet* query, int d, int k, int exclude_se
     if ((e = hipMemcpyAsync(list.p, retry.p, nr * sizeof(int), hipMemcpyDeviceToDevice, stream)) != hipSuccess ||
         (e = hipMemsetAsync(counters.p, 0, 2 * sizeof(int), stream)) != hipSuccess)
       return fail("KNN retry setup", e);
-    for (int q0 = 0, batch = batch_for(kp); q0 < nr; q0 += batch) {
+    for (int q0 = 0, batch = batch_for(kp, nr); q0 < nr; q0 += batch) {
       const int nq = std::min(batch, nr - q0);
       if ((e = launch_pass(pass, kp, list.p + q0, 0, nq, stream)) != hipSuccess) return fail("KNN retry launch", e);
     }

@@ -13,6 +13,7 @@ reference's argument errors, and a large input checked on sampled rows
 against a direct CPU computation.
 """
 
+import ctypes as C
 import sys
 
 import numpy as np
@@ -368,3 +369,38 @@ def test_query_errors(hip):
     with pytest.raises(_lib.HipBackendError, match="k exceeds"):
         hip.exact_query_knn(ref, ref[:3], 21)
     _check_query(hip.exact_query_knn(ref, ref[:3], 20), ref, ref[:3], 20)
+
+
+# Row widths at the edges of the scan's chunk counts (16, 32, 52, 64, 96, 128
+# dimensions) and one past them, and the finalize's load widths: d a multiple
+# of 4, of 2 and odd, with the device matrix 16, 8 and 4 bytes aligned.
+@pytest.mark.parametrize("offset", [0, 2, 1])
+@pytest.mark.parametrize("d", [1, 16, 17, 32, 33, 50, 52, 53, 64, 65, 96, 97, 128])
+def test_row_widths_and_alignments(hip, d, offset):
+    from fastembedr_amd.device import DeviceBuffer
+
+    _say(f"case: n=777 d={d} k=21, matrix {4 * offset} bytes past an aligned address")
+    n, k = 777, 21
+    x = np.random.default_rng(d).normal(size=(n, d)).astype(np.float32)
+    dev = DeviceBuffer.from_host(np.concatenate([np.zeros(offset, np.float32), x.ravel()]))
+    idx = np.empty((k, n), np.int32)
+    dist = np.empty((k, n), np.float32)
+    rc = _lib.load().fastembedr_hip_knn_exact(C.c_void_p(dev.address + 4 * offset), n, d, 0, k, 1, 1,
+                                              C.c_void_p(idx.ctypes.data), C.c_void_p(dist.ctypes.data), 0, None)
+    _lib.check(rc, "knn_exact")
+    ref_i, ref_d = knn_oracle.exact_knn(x, k)
+    np.testing.assert_array_equal(idx.T - 1, ref_i)
+    np.testing.assert_allclose(dist.T, ref_d, rtol=DIST_RTOL, atol=1e-30)
+
+
+# Cuts of a row's buffer where one value straddles the cut: m rows at exactly
+# one distance from every other (one-hot rows), more and fewer of them than
+# the first pass keeps, among far rows.
+@pytest.mark.parametrize("m,k", [(40, 15), (100, 15), (128, 30), (128, 90)])
+def test_cut_through_equal_distances(hip, m, k):
+    _say(f"case: {m} one-hot rows, k={k}")
+    rng = np.random.default_rng(m)
+    x = np.zeros((m + 900, 128), np.float32)
+    x[np.arange(m), np.arange(m)] = 1.0
+    x[m:] = 40.0 + rng.normal(size=(900, 128))
+    _check(hip.exact_knn(x, k), x, k)
