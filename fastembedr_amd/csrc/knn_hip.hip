@@ -227,66 +227,275 @@ constexpr int kProjDim = kKnnMaxDim;
 // the rest covers the fp64 projection and the basis' departure from exact
 // orthonormality (both below 1e-12 relative).
 constexpr int kProjSlack = 5;
-constexpr int kCovTile = 32;
-constexpr int kCovRows = 64;  // sample rows staged per step
+constexpr int kCovTile = 64;
+constexpr int kCovRows = 32;    // sample rows staged per step
+// Parts of the covariance's sample, each its own workgroups: enough for about
+// 1500 of them (six per CU), at most 16 (784 columns; one from 3500 on, where
+// the tiles alone are that many and a part takes 8 d^2 bytes).
+inline int knn_cov_parts(int d) {
+  const long long tiles = (d + 63) / 64;
+  return static_cast<int>(std::max(1ll, std::min(16ll, 1500 / (tiles * (tiles + 1) / 2))));
+}
+constexpr int kProjPanel = 16;  // columns orthonormalised together
 constexpr int kProjRows = 64;
 constexpr int kProjChunk = 32;
 
-// One 32 x 32 tile (bi, bj), bi <= bj, of the covariance of the centred
-// sample rows s * stride (s < m), fp64, mirrored into the lower tile.  Each
-// thread owns a 2 x 2 block of the tile.
+// One 64 x 64 tile (bi, bj), bi <= bj, of the covariance of the centred
+// sample rows s * stride, s in part blockIdx.z of [0, m), fp64, to
+// part[blockIdx.z].  Each thread owns a 4 x 4 block of the tile (8 LDS reads
+// per 16 FMAs; 2 x 2 blocks of 32 x 32 tiles read 4 per 4), and the parts give
+// a 784-column sample 91 x 16 workgroups instead of 325 with 312 steps each:
+// 2.4 -> 0.8 ms at 20,000 x 784.
 __global__ __launch_bounds__(256) void k_knn_cov(const float* __restrict__ x, Strides st, int d,
                                                  const double* __restrict__ mean, int m, long long stride,
-                                                 double* __restrict__ cov) {
+                                                 double* __restrict__ part) {
   const int bi = static_cast<int>(blockIdx.y), bj = static_cast<int>(blockIdx.x);
   if (bj < bi) return;  // whole block
   __shared__ double a[kCovRows][kCovTile + 1];
   __shared__ double b[kCovRows][kCovTile + 1];
   const int tid = static_cast<int>(threadIdx.x);
   const int ti = tid / 16, tj = tid % 16;
-  double acc00 = 0.0, acc01 = 0.0, acc10 = 0.0, acc11 = 0.0;
-  for (int s0 = 0; s0 < m; s0 += kCovRows) {
+  const int per = (m + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
+  const int m0 = static_cast<int>(blockIdx.z) * per, m1 = min(m, m0 + per);
+  double acc[4][4] = {};
+  for (int s0 = m0; s0 < m1; s0 += kCovRows) {
+#pragma unroll
     for (int e = tid; e < kCovRows * kCovTile; e += 256) {
       const int r = e / kCovTile, c = e % kCovTile;
       const int s = s0 + r;
       const int ca = bi * kCovTile + c, cb = bj * kCovTile + c;
       const long long row = static_cast<long long>(s) * stride;
-      a[r][c] = s < m && ca < d ? static_cast<double>(x[st.at(row, ca)]) - mean[ca] : 0.0;
-      b[r][c] = s < m && cb < d ? static_cast<double>(x[st.at(row, cb)]) - mean[cb] : 0.0;
+      a[r][c] = s < m1 && ca < d ? static_cast<double>(x[st.at(row, ca)]) - mean[ca] : 0.0;
+      b[r][c] = s < m1 && cb < d ? static_cast<double>(x[st.at(row, cb)]) - mean[cb] : 0.0;
     }
     __syncthreads();
+#pragma unroll 4
     for (int r = 0; r < kCovRows; ++r) {
-      const double a0 = a[r][2 * ti], a1 = a[r][2 * ti + 1];
-      const double b0 = b[r][2 * tj], b1 = b[r][2 * tj + 1];
-      acc00 = fma(a0, b0, acc00);
-      acc01 = fma(a0, b1, acc01);
-      acc10 = fma(a1, b0, acc10);
-      acc11 = fma(a1, b1, acc11);
+      double av[4], bv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        av[u] = a[r][ti + 16 * u];  // 16 apart: the lanes' reads fall in distinct banks
+        bv[u] = b[r][tj + 16 * u];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) acc[u][w] = fma(av[u], bv[w], acc[u][w]);
     }
     __syncthreads();
   }
-  const double v[2][2] = {{acc00, acc01}, {acc10, acc11}};
-  for (int u = 0; u < 2; ++u) {
-    for (int w = 0; w < 2; ++w) {
-      const int i = bi * kCovTile + 2 * ti + u, j = bj * kCovTile + 2 * tj + w;
-      if (i < d && j < d) {
-        cov[static_cast<long long>(i) * d + j] = v[u][w];
-        cov[static_cast<long long>(j) * d + i] = v[u][w];
-      }
+  double* const out = part + static_cast<long long>(blockIdx.z) * d * d;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int i = bi * kCovTile + ti + 16 * u, j = bj * kCovTile + tj + 16 * w;
+      if (i < d && j < d) out[static_cast<long long>(i) * d + j] = acc[u][w];
     }
   }
 }
 
-// y = cov q (d x d times d x kProjDim, row-major, fp64).  One block per row
-// of y, one thread per column.
+// The parts added in order, mirrored into the lower tiles; result in part 0.
+__global__ __launch_bounds__(256) void k_knn_cov_sum(double* __restrict__ part, int d, int parts) {
+  const int j = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+  const int i = static_cast<int>(blockIdx.y);
+  if (j >= d || j / kCovTile < i / kCovTile) return;
+  const long long at = static_cast<long long>(i) * d + j;
+  double s = 0.0;
+  for (int z = 0; z < parts; ++z) s += part[static_cast<long long>(z) * d * d + at];
+  part[at] = s;
+  if (j / kCovTile > i / kCovTile) part[static_cast<long long>(j) * d + i] = s;
+}
+
+// y = cov q (d x d times d x kProjDim, q row-major, y column-major, fp64).
+// One block per four rows of y, one thread per column.
 __global__ __launch_bounds__(kProjDim) void k_knn_cov_times(const double* __restrict__ cov,
                                                             const double* __restrict__ q, int d,
                                                             double* __restrict__ y) {
-  const long long i = blockIdx.x;
+  const long long i0 = 4ll * blockIdx.x;
   const int j = static_cast<int>(threadIdx.x);
-  double s = 0.0;
-  for (int c = 0; c < d; ++c) s = fma(cov[i * d + c], q[static_cast<long long>(c) * kProjDim + j], s);
-  y[i * kProjDim + j] = s;
+  const long long i1 = min(i0 + 1, d - 1ll), i2 = min(i0 + 2, d - 1ll), i3 = min(i0 + 3, d - 1ll);
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll 8
+  for (int c = 0; c < d; ++c) {
+    const double v = q[static_cast<long long>(c) * kProjDim + j];
+    s0 = fma(cov[i0 * d + c], v, s0);
+    s1 = fma(cov[i1 * d + c], v, s1);
+    s2 = fma(cov[i2 * d + c], v, s2);
+    s3 = fma(cov[i3 * d + c], v, s3);
+  }
+  double* const col = y + static_cast<long long>(j) * d;
+  const double out[4] = {s0, s1, s2, s3};
+  for (int u = 0; u < 4 && i0 + u < d; ++u) col[i0 + u] = out[u];
+}
+
+// Element i of a fixed stream of standard normals: SplitMix64 of the index,
+// then Box-Muller.
+__device__ __forceinline__ double proj_normal(unsigned long long i) {
+  auto mix = [](unsigned long long v) {
+    unsigned long long z = 0x6b6e6e70726f6aull + v * 0x9e3779b97f4a7c15ull;
+    z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+    z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+    z ^= z >> 31;
+    return (static_cast<double>(z >> 11) + 0.5) * 0x1.0p-53;
+  };
+  return sqrt(-2.0 * log(mix(2 * i + 1))) * cos(6.283185307179586 * mix(2 * i + 2));
+}
+
+__global__ __launch_bounds__(256) void k_knn_proj_random(double* __restrict__ q, long long count) {
+  const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < count) q[i] = proj_normal(static_cast<unsigned long long>(i));
+}
+
+// Sum over the workgroup of one value per thread, in every thread.
+template <int THREADS>
+__device__ __forceinline__ double block_sum(double v, double* scratch) {
+  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  __syncthreads();  // scratch may still be read
+  if ((threadIdx.x & (kWave - 1)) == 0) scratch[threadIdx.x / kWave] = v;
+  __syncthreads();
+  v = 0.0;
+  for (int w = 0; w < THREADS / kWave; ++w) v += scratch[w];
+  return v;
+}
+
+// Orthonormal columns of y (column-major, d x kProjDim), a panel of
+// kProjPanel columns at a time: the panel's components along the finished
+// columns are taken out (k_knn_proj_coef, k_knn_proj_update), its own columns
+// are orthonormalised (k_knn_proj_panel), and both are done a second time,
+// which removes what cancellation in the first left (block classical
+// Gram-Schmidt, twice).  On the host the same work, column by column, took
+// 130 ms for 784 columns.
+//
+// coef[k * kProjPanel + c] = y_k . y_(p0 + c) for the finished columns k < p0
+// (block k), and the squared norms of the panel's columns (blocks p0 + c) to
+// norms when wanted.
+__global__ __launch_bounds__(256) void k_knn_proj_coef(const double* __restrict__ y, int d, int p0,
+                                                       double* __restrict__ coef, double* __restrict__ norms) {
+  __shared__ double scratch[4];
+  const int k = static_cast<int>(blockIdx.x);
+  const int tid = static_cast<int>(threadIdx.x);
+  const double* const panel = y + static_cast<long long>(p0) * d;
+  if (k < p0) {
+    const double* const col = y + static_cast<long long>(k) * d;
+    double s[kProjPanel] = {};
+    for (int i = tid; i < d; i += 256) {
+      const double v = col[i];
+#pragma unroll
+      for (int c = 0; c < kProjPanel; ++c) s[c] = fma(v, panel[static_cast<long long>(c) * d + i], s[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < kProjPanel; ++c) {
+      const double t = block_sum<256>(s[c], scratch);
+      if (tid == 0) coef[k * kProjPanel + c] = t;
+    }
+  } else {
+    const double* const col = panel + static_cast<long long>(k - p0) * d;
+    double s = 0.0;
+    for (int i = tid; i < d; i += 256) s = fma(col[i], col[i], s);
+    s = block_sum<256>(s, scratch);
+    if (tid == 0) norms[k - p0] = s;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_knn_proj_update(double* __restrict__ y, int d, int p0,
+                                                         const double* __restrict__ coef) {
+  const int i = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+  const int c = static_cast<int>(blockIdx.y);
+  if (i >= d) return;
+  double v = y[static_cast<long long>(p0 + c) * d + i];
+#pragma unroll 8
+  for (int k = 0; k < p0; ++k) v = fma(-coef[k * kProjPanel + c], y[static_cast<long long>(k) * d + i], v);
+  y[static_cast<long long>(p0 + c) * d + i] = v;
+}
+
+// The panel's own columns, one workgroup of 16 waves: for each column, the
+// earlier columns' components are taken out `passes` times (a wave per dot
+// product), then it is scaled to length 1.  A column left without a direction
+// of its own (`norms`: its squared length before anything was taken out; the
+// data's rank below kProjDim) is redrawn at random and made orthogonal to all
+// finished columns, and is zero if that fails eight times (a zero column
+// keeps Q contractive).
+//
+// Bound by the latency of its serial chain (16 columns, each a few reductions
+// over the workgroup), so the panel stays in LDS where it fits (STAGED:
+// kProjPanel d doubles, d up to kPanelStaged): 64 us a launch at 784 columns,
+// 127 us reading it through L2.
+constexpr int kPanelThreads = 1024;
+constexpr int kPanelStaged = 1152;  // 144 KB of LDS
+
+template <bool STAGED>
+__global__ __launch_bounds__(kPanelThreads) void k_knn_proj_panel(double* __restrict__ y, int d, int p0, int passes,
+                                                                  const double* __restrict__ norms) {
+  extern __shared__ double staged[];
+  __shared__ double coef[kProjDim];
+  __shared__ double scratch[kPanelThreads / kWave];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  constexpr int kWaves = kPanelThreads / kWave;
+  double* const home = y + static_cast<long long>(p0) * d;
+  auto column = [&](int c) -> double* {
+    if constexpr (STAGED) return staged + c * d;
+    else return home + static_cast<long long>(c) * d;
+  };
+  if constexpr (STAGED) {
+    for (int e = tid; e < kProjPanel * d; e += kPanelThreads) staged[e] = home[e];
+  }
+  for (int c = 0; c < kProjPanel; ++c) {
+    double* const col = column(c);
+    bool redrawn = false;  // earlier panels' columns are taken out as well
+    int times = passes;
+    double before = norms != nullptr ? norms[c] : 1.0;
+    for (int tries = 0;; ++tries) {
+      for (int t = 0; t < times; ++t) {
+        __syncthreads();  // the column is written, coef is read
+        auto dot = [&](const double* other, int at) {
+          double s = 0.0;
+#pragma unroll 8
+          for (int i = lane; i < d; i += kWave) s = fma(other[i], col[i], s);
+          for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_xor(s, off);
+          if (lane == 0) coef[at] = s;
+        };
+        for (int k = wave; k < c; k += kWaves) dot(column(k), p0 + k);
+        if (redrawn)
+          for (int k = wave; k < p0; k += kWaves) dot(y + static_cast<long long>(k) * d, k);
+        __syncthreads();
+        for (int i = tid; i < d; i += kPanelThreads) {
+          double v = col[i];
+#pragma unroll 4
+          for (int k = 0; k < c; ++k) v = fma(-coef[p0 + k], column(k)[i], v);
+          if (redrawn)
+            for (int k = 0; k < p0; ++k) v = fma(-coef[k], y[static_cast<long long>(k) * d + i], v);
+          col[i] = v;
+        }
+      }
+      double s = 0.0;
+      for (int i = tid; i < d; i += kPanelThreads) s = fma(col[i], col[i], s);  // the thread's own values
+      const double after = block_sum<kPanelThreads>(s, scratch);
+      if ((after > 1e-20 * before && after > 0.0 && isfinite(after)) || tries == 8) {
+        const double inv = tries == 8 ? 0.0 : 1.0 / sqrt(after);
+        for (int i = tid; i < d; i += kPanelThreads) col[i] = tries == 8 ? 0.0 : col[i] * inv;
+        break;
+      }
+      for (int i = tid; i < d; i += kPanelThreads)
+        col[i] = proj_normal((static_cast<unsigned long long>(kProjDim + p0 + c) * 9 + tries) * d + i);
+      redrawn = true;
+      times = 2;
+      before = 1.0;
+    }
+  }
+  if constexpr (STAGED) {
+    __syncthreads();
+    for (int e = tid; e < kProjPanel * d; e += kPanelThreads) home[e] = staged[e];
+  }
+}
+
+// q (row-major) = y (column-major).
+__global__ __launch_bounds__(256) void k_knn_proj_transpose(const double* __restrict__ y, int d,
+                                                            double* __restrict__ q) {
+  const long long e = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  if (e >= static_cast<long long>(d) * kProjDim) return;
+  q[e] = y[(e % kProjDim) * d + e / kProjDim];
 }
 
 // Projected rows: xc row = fl32(Q^T (x - mean)) (fp64 sums), zero in
@@ -1382,83 +1591,52 @@ struct KnnSet {
   int on_device;
 };
 
-// Uniform 64-bit stream (SplitMix64) and standard normals from it
-// (Box-Muller), for the power iterations' fixed start.
-struct ProjRng {
-  std::uint64_t s;
-  std::uint64_t next() {
-    std::uint64_t z = (s += 0x9e3779b97f4a7c15ull);
-    z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
-    z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-    return z ^ (z >> 31);
-  }
-  double uniform() { return (static_cast<double>(next() >> 11) + 0.5) * 0x1.0p-53; }
-  double normal() { return std::sqrt(-2.0 * std::log(uniform())) * std::cos(6.283185307179586 * uniform()); }
-};
-
-// Orthonormal columns for the d x kProjDim row-major matrix y (modified
-// Gram-Schmidt, two passes, fp64).  A column left without a direction of its
-// own (the data's rank below kProjDim) is redrawn at random.
-void proj_orthonormalize(std::vector<double>& y, int d, ProjRng& rng) {
-  constexpr int m = kProjDim;
-  for (int j = 0; j < m; ++j) {
-    for (;;) {
-      double before = 0.0;
-      for (int i = 0; i < d; ++i) before += y[static_cast<std::size_t>(i) * m + j] * y[static_cast<std::size_t>(i) * m + j];
-      for (int pass = 0; pass < 2; ++pass) {
-        for (int k = 0; k < j; ++k) {
-          double dot = 0.0;
-          for (int i = 0; i < d; ++i) dot += y[static_cast<std::size_t>(i) * m + k] * y[static_cast<std::size_t>(i) * m + j];
-          for (int i = 0; i < d; ++i) y[static_cast<std::size_t>(i) * m + j] -= dot * y[static_cast<std::size_t>(i) * m + k];
-        }
-      }
-      double after = 0.0;
-      for (int i = 0; i < d; ++i) after += y[static_cast<std::size_t>(i) * m + j] * y[static_cast<std::size_t>(i) * m + j];
-      if (after > 1e-20 * before && after > 0.0 && std::isfinite(after)) {
-        const double inv = 1.0 / std::sqrt(after);
-        for (int i = 0; i < d; ++i) y[static_cast<std::size_t>(i) * m + j] *= inv;
-        break;
-      }
-      for (int i = 0; i < d; ++i) y[static_cast<std::size_t>(i) * m + j] = rng.normal();
-    }
-  }
-}
-
 // Q (d x kProjDim, orthonormal columns, on the device) spanning the leading
 // principal directions of the rows of x: covariance of up to kProjSample
 // evenly spaced rows, then kProjIters block power iterations from a fixed
-// random start, each followed by an orthonormalisation on the host.
+// random start, each followed by an orthonormalisation.  Stream-ordered;
+// cov, y_dev and coef are the caller's scratch (knn_cov_parts(d) d d, d kProjDim
+// and kProjDim kProjPanel + kProjPanel values).
 constexpr int kProjSample = 32768;
 constexpr int kProjIters = 4;
 
-hipError_t knn_projection_basis(const float* x, Strides st, int n, int d, const double* mean, double* q_dev,
-                                hipStream_t stream) {
+hipError_t knn_projection_basis(const float* x, Strides st, int n, int d, const double* mean, double* cov,
+                                double* y_dev, double* coef, double* q_dev, hipStream_t stream) {
   const int m = std::min(n, kProjSample);
   const long long stride = std::max(1, n / m);
-  DevBuf<double> cov, y_dev;
-  hipError_t e;
-  if ((e = cov.alloc(static_cast<std::size_t>(d) * d)) != hipSuccess ||
-      (e = y_dev.alloc(static_cast<std::size_t>(d) * kProjDim)) != hipSuccess)
-    return e;
   const int tiles = (d + kCovTile - 1) / kCovTile;
-  k_knn_cov<<<dim3(tiles, tiles), 256, 0, stream>>>(x, st, d, mean, m, stride, cov.p);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  std::vector<double> q(static_cast<std::size_t>(d) * kProjDim);
-  ProjRng rng{0x6b6e6e70726f6aull};
-  for (double& v : q) v = rng.normal();
-  proj_orthonormalize(q, d, rng);
-  const std::size_t bytes = q.size() * sizeof(double);
-  for (int it = 0; it < kProjIters; ++it) {
-    if ((e = hipMemcpyAsync(q_dev, q.data(), bytes, hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
-    k_knn_cov_times<<<d, kProjDim, 0, stream>>>(cov.p, q_dev, d, y_dev.p);
-    if ((e = hipGetLastError()) != hipSuccess ||
-        (e = hipMemcpyAsync(q.data(), y_dev.p, bytes, hipMemcpyDeviceToHost, stream)) != hipSuccess ||
-        (e = hipStreamSynchronize(stream)) != hipSuccess)
-      return e;
-    proj_orthonormalize(q, d, rng);
+  const unsigned int col_blocks = static_cast<unsigned int>((d + 255) / 256);
+  const long long values = static_cast<long long>(d) * kProjDim;
+  const unsigned int value_blocks = static_cast<unsigned int>((values + 255) / 256);
+  double* const norms = coef + kProjDim * kProjPanel;
+  const std::size_t panel_lds = sizeof(double) * kProjPanel * static_cast<std::size_t>(d);
+  if (d <= kPanelStaged) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_knn_proj_panel<true>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(panel_lds));
+    if (e != hipSuccess) return e;
   }
-  if ((e = hipMemcpyAsync(q_dev, q.data(), bytes, hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
-  return hipStreamSynchronize(stream);
+  const int parts = knn_cov_parts(d);
+  k_knn_cov<<<dim3(tiles, tiles, parts), 256, 0, stream>>>(x, st, d, mean, m, stride, cov);
+  k_knn_cov_sum<<<dim3(col_blocks, d), 256, 0, stream>>>(cov, d, parts);
+  k_knn_proj_random<<<value_blocks, 256, 0, stream>>>(q_dev, values);
+  for (int it = 0; it < kProjIters; ++it) {
+    k_knn_cov_times<<<(d + 3) / 4, kProjDim, 0, stream>>>(cov, q_dev, d, y_dev);
+    for (int p0 = 0; p0 < kProjDim; p0 += kProjPanel) {
+      for (int round = 0; round < 2; ++round) {
+        const int blocks = p0 + (round == 0 ? kProjPanel : 0);
+        if (blocks > 0) k_knn_proj_coef<<<blocks, 256, 0, stream>>>(y_dev, d, p0, coef, norms);
+        if (p0 > 0) k_knn_proj_update<<<dim3(col_blocks, kProjPanel), 256, 0, stream>>>(y_dev, d, p0, coef);
+        const int passes = round == 0 ? 2 : 1;
+        const double* const before = round == 0 ? norms : nullptr;
+        if (d <= kPanelStaged)
+          k_knn_proj_panel<true><<<1, kPanelThreads, panel_lds, stream>>>(y_dev, d, p0, passes, before);
+        else
+          k_knn_proj_panel<false><<<1, kPanelThreads, 0, stream>>>(y_dev, d, p0, passes, before);
+      }
+    }
+    k_knn_proj_transpose<<<value_blocks, 256, 0, stream>>>(y_dev, d, q_dev);
+  }
+  return hipGetLastError();
 }
 
 // The whole search: references `ref`, queries `query` (null: the references
@@ -1480,7 +1658,7 @@ int knn_run(const KnnSet& ref, const KnnSet* query, int d, int k, int exclude_se
   hipStream_t stream = nullptr;
   hipError_t e;
   DevBuf<float> xr_dev, xq_dev, xc, nrm, xcq, nrmq, dist_dev;
-  DevBuf<double> partial, mean, basis;
+  DevBuf<double> partial, mean, basis, cov, proj_y, proj_coef;
   DevBuf<unsigned int> nrm_max;
   DevBuf<int> idx_dev, retry, counters;
   auto upload = [&](const KnnSet& set, DevBuf<float>& dev, const float*& out) -> hipError_t {
@@ -1553,8 +1731,12 @@ int knn_run(const KnnSet& ref, const KnnSet* query, int d, int k, int exclude_se
   k_knn_col_partials<<<pblocks, kPrepThreads, 0, stream>>>(xr, n, d, str, rows_per, partial.p);
   k_knn_col_means<<<(d + kWave - 1) / kWave, kPrepThreads, 0, stream>>>(partial.p, pblocks, d, n, mean.p);
   if (project) {
-    if ((e = basis.alloc(static_cast<std::size_t>(d) * kProjDim)) != hipSuccess) return fail("hipMalloc(KNN basis)", e);
-    if ((e = knn_projection_basis(xr, str, n, d, mean.p, basis.p, stream)) != hipSuccess)
+    const std::size_t dd = static_cast<std::size_t>(d);
+    if ((e = basis.alloc(dd * kProjDim)) != hipSuccess || (e = cov.alloc(knn_cov_parts(d) * dd * dd)) != hipSuccess ||
+        (e = proj_y.alloc(dd * kProjDim)) != hipSuccess ||
+        (e = proj_coef.alloc(kProjDim * kProjPanel + kProjPanel)) != hipSuccess)
+      return fail("hipMalloc(KNN basis)", e);
+    if ((e = knn_projection_basis(xr, str, n, d, mean.p, cov.p, proj_y.p, proj_coef.p, basis.p, stream)) != hipSuccess)
       return fail("KNN projection basis", e);
     k_knn_project<<<(n_pad + kProjRows - 1) / kProjRows, 256, 0, stream>>>(xr, n, n_pad, d, str, P, mean.p, basis.p,
                                                                           xc.p, nrm.p, nrm_max.p, counters.p + 2);

@@ -404,3 +404,14 @@ def test_cut_through_equal_distances(hip, m, k):
     x[np.arange(m), np.arange(m)] = 1.0
     x[m:] = 40.0 + rng.normal(size=(900, 128))
     _check(hip.exact_knn(x, k), x, k)
+
+
+# The projection's basis: rank far below its 128 columns (the missing ones are
+# redrawn), one column past a panel staged in LDS, and widths off the
+# covariance's 64-column tiles; parts of its sample from 16 down to 1.
+@pytest.mark.parametrize("n,d,rank", [(900, 129, 3), (700, 193, 40), (400, 1152, 20), (400, 1153, 20), (300, 4000, 12)])
+def test_projection_basis_shapes(hip, n, d, rank):
+    _say(f"case: projected rows n={n} d={d} rank={rank}")
+    rng = np.random.default_rng(d)
+    x = (rng.normal(size=(n, rank)) @ rng.normal(size=(rank, d))).astype(np.float32)
+    _check(hip.exact_knn(x, 12), x, 12)
