@@ -2011,7 +2011,7 @@ int fastembedr_hip_tsne_kl(fastembedr_hip_tsne* s, double* kl) { return fastembe
 
 int fastembedr_hip_tsne_kl_rows(fastembedr_hip_tsne* s, double* kl, double* row_costs) {
   if (!valid_state_args(s) || kl == nullptr) return 1;
-  const int zb = fehip::exact_blocks_for(s->n);
+  const int zb = fehip::exact_z_blocks_for(s->n);
   std::vector<double> part(static_cast<std::size_t>(std::max(zb, 1024)));
   if (!hip_ok(fehip::launch_exact_z_double(s->y_a(), s->n, s->dpartial, s->stream), "exact_z launch") ||
       !hip_ok(hipMemcpyAsync(part.data(), s->dpartial, zb * sizeof(double), hipMemcpyDeviceToHost, s->stream),

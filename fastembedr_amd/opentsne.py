@@ -324,15 +324,18 @@ def opentsne_knn(indices, distances=None, n_neighbors: int | None = None, perple
                     done += step_n
                     left -= step_n
                     if (record_costs or verbose) and (done % 50 == 0 or done == total):
-                        costs.append(sess.kl())
+                        # the final layout's rows come with its cost
+                        if record_costs and done == total:
+                            cost, row_costs = sess.kl_rows()
+                        else:
+                            cost = sess.kl()
+                        costs.append(cost)
                         its.append(done)
                         if verbose:
                             print(f"Iteration {done}: error is {costs[-1]}")
             out = sess.y
             itercosts = np.asarray(costs)
             iters = np.asarray(its, np.int32)
-            if record_costs:
-                _, row_costs = sess.kl_rows()
         finally:
             sess.close()
     else:

@@ -234,6 +234,27 @@ def test_kl_matches_oracle(hip, oracle_mod, mid_problem):
     assert np.abs(rows_run - ref_rows_run).max() <= 1e-6 * np.abs(ref_rows_run).max()
 
 
+@pytest.mark.parametrize("n", [17, 255, 256, 257, 511, 513, 1030])
+@pytest.mark.parametrize("spread", [0.0, 1.0, 1e19])
+def test_kl_tile_edges(hip, oracle_mod, n, spread):
+    """The normaliser's 256-point tiles (alone, partial, diagonal) and rows of
+    the KL shorter and longer than its 16 lanes; all points at one place, an
+    ordinary layout, and one whose squared distances overflow fp32."""
+    _say(f"case: exact KL, n={n} spread={spread}")
+    k = min(n - 1, 40)
+    x, labels, idx, dist = small_problem(n=n, dim=6, k=k, components=2, seed=n)
+    y = (np.random.default_rng(n).standard_normal((n, 2)) * 3 * spread).astype(np.float32)
+    with hip.TsneSession(idx, dist, perplexity=5.0, index_offset=1) as s:
+        s.set_state(y)
+        kl, rows = s.kl_rows()
+        P = oracle_mod.OracleP.wrap(*s.csr())
+    ref, ref_rows = P.kl(y, threads=2, row_costs=True)
+    # the fp32 rounding of the normaliser may fall the other way: 2^-24 of the
+    # terms' mass 1 (and of the logarithms' sum)
+    assert abs(kl - ref) <= 2e-7 * max(1.0, abs(ref))
+    assert np.abs(rows - ref_rows).max() <= 2e-7 * max(np.abs(ref_rows).max(), 1.0 / n)
+
+
 def _one_shot(fn_name, idx, dist, init, n_early, n_norm, device=False, shape=None):
     lib = _lib.load()
     n, k = shape if device else idx.shape
