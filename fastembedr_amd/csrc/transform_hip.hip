@@ -739,6 +739,142 @@ __global__ __launch_bounds__(kLaneThreads) void k_transform_grid_lanes(
   }
 }
 
+// ---- sampled and exact modes with L lanes per query ------------------------------
+// As k_transform_grid_lanes: the neighbours are dealt to the group's lanes
+// and stay in their registers, the update is computed by every lane.  The
+// repulsion's samples are dealt to the lanes in runs of ceil(samples / L)
+// consecutive draws, so that the group takes exactly the reference's draws;
+// a lane enters the query's xorshift sequence at its own run's start, which
+// is a linear map of the iteration's state over GF(2) (the generator's step
+// is one), applied as eight table lookups of four bits each.  In exact mode
+// the lanes stride over the references.  One pass collects sum q and
+// sum q^2 d (the reference's two passes draw the samples twice), added
+// across the lanes: another order of the fp64 sums than the reference's.
+//
+// Bound by the scattered 16-byte reads of the sampled references (a cache
+// line each); one thread per query left a call of 12,345 queries with 193
+// waves for 1,024 SIMDs and took 12.3 ms for 250 iterations of 256 samples.
+constexpr int kJumpStride = 129;  // table words per lane position (8 x 16, padded off one bank)
+
+template <int L>
+__device__ __forceinline__ void build_jump_tables(std::uint32_t (&table)[L * kJumpStride], int run) {
+  const int tid = static_cast<int>(threadIdx.x);
+  // the images of the 32 single bits after lane * run steps, parked in the
+  // first 32 words of the lane position's table
+  for (int e = tid; e < L * 32; e += kLaneThreads) {
+    std::uint32_t s = 1u << (e % 32);
+    for (int t = (e / 32) * run; t > 0; --t) (void)draw_index(s, 1);
+    table[(e / 32) * kJumpStride + e % 32] = s;
+  }
+  __syncthreads();
+  // then the 16 combinations of each group of four bits: L * 8 groups, whole
+  // lane positions per thread set, read before they are overwritten
+  constexpr int kGroups = (L * 8 + kLaneThreads - 1) / kLaneThreads;
+  std::uint32_t bits[kGroups][4];
+  for (int r = 0; r < kGroups; ++r) {
+    const int e = tid + r * kLaneThreads;
+    for (int b = 0; b < 4; ++b)
+      bits[r][b] = e < L * 8 ? table[(e / 8) * kJumpStride + (e % 8) * 4 + b] : 0u;
+  }
+  __syncthreads();
+  for (int r = 0; r < kGroups; ++r) {
+    const int e = tid + r * kLaneThreads;
+    if (e < L * 8) {
+      for (int v = 0; v < 16; ++v)
+        table[(e / 8) * kJumpStride + (e % 8) * 16 + v] = (v & 1 ? bits[r][0] : 0u) ^ (v & 2 ? bits[r][1] : 0u) ^
+                                                         (v & 4 ? bits[r][2] : 0u) ^ (v & 8 ? bits[r][3] : 0u);
+    }
+  }
+  __syncthreads();
+}
+
+template <int MODE, int L, int MAXJ>
+__global__ __launch_bounds__(kLaneThreads) void k_transform_lanes(const double2* __restrict__ ref, int n_ref,
+                                                                  const int* __restrict__ idx_cm,
+                                                                  const double* __restrict__ p_cm, int nq, int k,
+                                                                  int offset, RunSchedule rs,
+                                                                  double2* __restrict__ y) {
+#pragma clang fp contract(off)
+  static_assert(MODE == kSampled || MODE == kExact, "the grid mode has its own kernel");
+  __shared__ std::uint32_t table[MODE == kSampled ? L * kJumpStride : 1];
+  const int run = (rs.samples + L - 1) / L;
+  if constexpr (MODE == kSampled) build_jump_tables<L>(table, run);
+  const long long gid = static_cast<long long>(blockIdx.x) * kLaneThreads + static_cast<long long>(threadIdx.x);
+  const int i = static_cast<int>(gid / L);
+  const int lane = static_cast<int>(threadIdx.x) & (L - 1);
+  // a group past the last query repeats the last one and writes nothing
+  const int qi = i < nq ? i : nq - 1;
+  double px[MAXJ], py[MAXJ], pj[MAXJ];
+#pragma unroll
+  for (int jj = 0; jj < MAXJ; ++jj) {
+    const int j = lane + jj * L;
+    px[jj] = 0.0;
+    py[jj] = 0.0;
+    pj[jj] = 0.0;
+    if (j < k) {
+      const std::size_t e = static_cast<std::size_t>(j) * nq + qi;
+      const double2 r = ref[idx_cm[e] - offset];
+      px[jj] = r.x;
+      py[jj] = r.y;
+      pj[jj] = p_cm[e];
+    }
+  }
+  double2 yi = y[qi];
+  double2 u = make_double2(0.0, 0.0);
+  double2 w = make_double2(1.0, 1.0);
+  const int mine = max(0, min(run, rs.samples - lane * run));  // draws of this lane's run
+  for (int it = 0; it < rs.total; ++it) {
+    const bool early = it < rs.early_iter;
+    double sq = 0.0, sx = 0.0, sy = 0.0;
+    auto add = [&](const double2& r) {
+      const double dx = yi.x - r.x;
+      const double dy = yi.y - r.y;
+      const double q = recip_ge1(1.0 + dx * dx + dy * dy);
+      const double q2 = q * q;
+      sq += q;
+      sx += q2 * dx;
+      sy += q2 * dy;
+    };
+    if constexpr (MODE == kSampled) {
+      const std::uint32_t s0 = query_state(rs.seed_base + 65537u * static_cast<std::uint32_t>(it + 1), qi);
+      std::uint32_t s = 0u;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) s ^= table[lane * kJumpStride + b * 16 + ((s0 >> (4 * b)) & 15u)];
+      int m = 0;
+      for (; m + 8 <= mine; m += 8) {
+        double2 r[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) r[t] = ref[draw_index(s, n_ref)];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) add(r[t]);
+      }
+      for (; m < mine; ++m) add(ref[draw_index(s, n_ref)]);
+    } else {
+#pragma unroll 4
+      for (int m = lane; m < rs.samples; m += L) add(ref[m]);
+    }
+    const double ex = early ? rs.early_exaggeration : rs.exaggeration;
+    double ax = 0.0, ay = 0.0;
+#pragma unroll
+    for (int jj = 0; jj < MAXJ; ++jj) {
+      if (lane + jj * L < k) {
+        const double dx = yi.x - px[jj];
+        const double dy = yi.y - py[jj];
+        const double q = recip_ge1(1.0 + dx * dx + dy * dy);
+        const double c = ex * pj[jj] * q;
+        ax += c * dx;
+        ay += c * dy;
+      }
+    }
+    const double inv = 1.0 / (DBL_MIN + group_sum<L>(sq));
+    const double gx = group_sum<L>(ax) - group_sum<L>(sx) * inv;
+    const double gy = group_sum<L>(ay) - group_sum<L>(sy) * inv;
+    update_query(gx, gy, early ? rs.initial_momentum : rs.final_momentum, rs.learning_rate, rs.max_grad, rs.max_step,
+                 yi, u, w);
+  }
+  if (i < nq && lane == 0) y[i] = yi;
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -1044,6 +1180,14 @@ hipError_t launch_grid_fields(const double2* ref, int n_ref, const GridGeo& g, c
   return hipGetLastError();
 }
 
+// Lanes per query of the sampled and exact modes: 16 from this many queries
+// on (1,024 waves, one per SIMD), else 64.  250 iterations of 256 samples of
+// 70,000 references, whole calls (one thread per query before): 200 queries
+// 12.1 -> 0.96 ms, 2,000 12.1 -> 1.16, 12,345 13.0 -> 4.2 (64 lanes 4.4),
+// 40,000 24.0 -> 11.1 (4 lanes 11.8); exact mode over 3,000 references: 3,000
+// queries 102 -> 2.6 ms, 20,000 104 -> 12.4 (4 lanes 27.4).
+constexpr int kLanes16Queries = 4096;
+
 hipError_t launch_run(int mode, const double2* ref, int n_ref, const int* idx, const double* p, int nq, int k,
                       int offset, const RunSchedule& rs, const double4* field, const GridGeo& g, double2* y,
                       unsigned long long* counter, hipStream_t st) {
@@ -1069,6 +1213,32 @@ hipError_t launch_run(int mode, const double2* ref, int n_ref, const int* idx, c
       lanes(std::integral_constant<int, 16>{}, I8{});
     } else {
       lanes(std::integral_constant<int, 32>{}, I8{});
+    }
+  } else if (mode != kGrid && k <= 256 && nq > 0) {
+    // lanes per query
+    const auto lanes = [&](auto tag_l, auto tag_j) {
+      constexpr int L = decltype(tag_l)::value;
+      constexpr int J = decltype(tag_j)::value;
+      const long long threads = static_cast<long long>(nq) * L;
+      const unsigned int lb = static_cast<unsigned int>((threads + kLaneThreads - 1) / kLaneThreads);
+      if (mode == kExact)
+        k_transform_lanes<kExact, L, J><<<lb, kLaneThreads, 0, st>>>(ref, n_ref, idx, p, nq, k, offset, rs, y);
+      else
+        k_transform_lanes<kSampled, L, J><<<lb, kLaneThreads, 0, st>>>(ref, n_ref, idx, p, nq, k, offset, rs, y);
+    };
+    using I4 = std::integral_constant<int, 4>;
+    using I16 = std::integral_constant<int, 16>;
+    using I64 = std::integral_constant<int, 64>;
+    if (nq >= kLanes16Queries) {
+      if (k <= 32)
+        lanes(I16{}, std::integral_constant<int, 2>{});
+      else
+        lanes(I16{}, I16{});
+    } else {
+      if (k <= 64)
+        lanes(I64{}, std::integral_constant<int, 1>{});
+      else
+        lanes(I64{}, I4{});
     }
   } else if (mode == kGrid) {
     k_transform_run<kGrid><<<blocks, kRunThreads, 0, st>>>(ref, n_ref, idx, p, nq, k, offset, rs, field, g, y,

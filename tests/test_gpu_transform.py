@@ -136,6 +136,24 @@ def test_transform_run_matches_oracle(hip, oracle_mod, qp, case):
     assert dev <= 1e-9 * scale
 
 
+@pytest.mark.parametrize("mode", ["sampled", "exact"])
+@pytest.mark.parametrize("nq,k,samples", [(1, 3, 1), (5, 1, 63), (130, 64, 65), (90, 65, 100), (70, 256, 256), (40, 257, 7),
+                                          (4095, 15, 33), (4096, 32, 16), (4099, 33, 17)])
+def test_transform_lane_widths(hip, oracle_mod, mode, nq, k, samples):
+    """Both lane widths of the run kernel (64 below 4,096 queries, 16 from
+    there on), their neighbour counts and the one-thread kernel past 256, and
+    sample counts off the lanes (runs of unequal length, lanes without any)."""
+    _say(f"case: transform lanes {mode}, nq={nq} k={k} samples={samples}")
+    ref, idx, dist = query_problem(n_ref=300, nq=nq, k=k, seed=nq + k)
+    kw = dict(perplexity=min(5.0, max(1.0, k / 3.0)), n_iter=12, learning_rate=0.1, exaggeration=1.5, seed=23)
+    thr = 100 if mode == "sampled" else 4096
+    y, cfg = _run(ref, idx, dist, exact_repulsion_threshold=thr, n_negatives=samples if mode == "sampled" else 300, **kw)
+    y_ref, exact = oracle_mod.transform_run(ref, idx, dist, threads=8, exact_threshold=thr,
+                                            n_negatives=samples if mode == "sampled" else 300, **kw)
+    assert bool(exact) == (mode == "exact")
+    assert np.abs(y - y_ref).max() <= 1e-9 * np.abs(y_ref).max()
+
+
 def test_transform_is_deterministic(hip, qp):
     ref, idx, dist = qp
     a, _ = _run(ref, idx, dist, n_iter=20, exact_repulsion_threshold=100, seed=3)
