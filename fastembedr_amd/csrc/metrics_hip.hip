@@ -12,7 +12,9 @@
 // continuity likewise, knn preservation = shared / (n k), mean neighbour rank
 // error = rank error / (n k).
 //
-// One workgroup per row: its squared distances in each space are formed in
+// Requests of up to kSelMaxK neighbours select them (k_structure_select); the
+// rows that it lists, larger requests and small n are sorted (k_structure_rows): one
+// workgroup per row, its squared distances in each space are formed in
 // fp64 with the reference's operation order (a sequential sum over columns of
 // the rounded squares, no fused multiply-add), so they are bit-identical to
 // the reference's; the (d2, index) pairs are sorted in LDS (bitonic), ranks
@@ -89,10 +91,12 @@ __device__ void rank_row(const double* __restrict__ x, int n, int p, int i, int 
 }
 
 // Dynamic LDS: key[m] (fp64), idx[m], high_rank[n], low_rank[n], high_order[kmax].
+// Row i = rows[block], or the block (null).
 // Row sums: sums[(i * nk + q) * 4 + {0: shared, 1: trust, 2: continuity, 3: rank error}].
 __global__ __launch_bounds__(kMetThreads) void k_structure_rows(const double* __restrict__ high, int p_high,
                                                                 const double* __restrict__ low, int p_low, int n,
                                                                 int m, const int* __restrict__ ks, int nk, int kmax,
+                                                                const int* __restrict__ rows,
                                                                 double* __restrict__ sums) {
   extern __shared__ double lds[];
   double* const key = lds;
@@ -101,7 +105,7 @@ __global__ __launch_bounds__(kMetThreads) void k_structure_rows(const double* __
   int* const low_rank = high_rank + n;
   int* const high_order = low_rank + n;
   __shared__ double part[4][kMetThreads / 64];
-  const int i = static_cast<int>(blockIdx.x);
+  const int i = rows != nullptr ? rows[blockIdx.x] : static_cast<int>(blockIdx.x);
   const int tid = static_cast<int>(threadIdx.x);
 
   rank_row(high, n, p_high, i, m, key, idx, high_rank);
@@ -142,6 +146,230 @@ __global__ __launch_bounds__(kMetThreads) void k_structure_rows(const double* __
       sums[(static_cast<long long>(i) * nk + q) * 4 + tid] = s;
     }
     __syncthreads();
+  }
+}
+
+// ---- small k: selection instead of sorting ---------------------------------------
+// The metrics need the k nearest in each space and those neighbours' ranks in
+// the other space, not whole orders.  A workgroup takes kSelRows rows; each
+// thread keeps its 1/512 of their distances in both spaces in registers (PER
+// of them per row and space).  Per row and space: a bound t with kmax to
+// kSelCand distances at or below it (bisection, one barrier a step), those
+// candidates ordered by (d2, index) by counting; then the rank of every
+// neighbour in the other space by counting the distances before its own
+// (compares and ballots).  The row itself and padding hold NaN, which no
+// comparison counts.  Rows that find no such bound (more than kSelCand equal
+// distances at the k-th place, infinities, NaN data) are listed for
+// k_structure_rows.  Sorting 8192 pairs twice a row in LDS took 11.6 ms at
+// 5,000 rows; two rows a workgroup halve the reads of the data from L2, which
+// bound this kernel.
+constexpr int kSelThreads = 512;
+constexpr int kSelRows = 2;
+constexpr int kSelCand = 128;
+// Counting takes kmax compares a distance: past this the sort is used (5,000
+// x 50: k = 5 1.1 ms, 15 1.3, 30 1.6, 64 2.3; sorting 11.9 for any k).
+constexpr int kSelMaxK = 64;
+// Below this many rows sorting is as fast (500 rows 0.21 ms against 0.28;
+// 1,500 rows 0.47 against 0.26).
+constexpr int kSelMinRows = 1025;
+
+struct SelRow {
+  double cand_d[2][kSelCand];
+  int cand_j[2][kSelCand];
+  int nb[2][kSelMaxK];        // neighbours in order, space 0 high, 1 low
+  double other[2][kSelMaxK];  // their squared distances in the other space
+  int rank[2][kSelMaxK];      // their ranks in the other space
+  int count[2];
+};
+
+static_assert(kMetMaxRows <= 10 * kSelThreads, "a thread keeps at most ten distances of a row and space");
+
+template <int PER>
+__global__ __launch_bounds__(kSelThreads) void k_structure_select(const double* __restrict__ high, int p_high,
+                                                                  const double* __restrict__ low, int p_low, int n,
+                                                                  const int* __restrict__ ks, int nk, int kmax,
+                                                                  double* __restrict__ sums, int* __restrict__ todo) {
+  __shared__ SelRow row;
+  __shared__ double red[2][2][kSelThreads / 64];
+  __shared__ int cnt[2][kSelThreads / 64];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & 63, wave = tid / 64;
+  constexpr int kWaves = kSelThreads / 64;
+  const int i0 = static_cast<int>(blockIdx.x) * kSelRows;
+
+  double d[kSelRows][2][PER];
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    const int j = tid + e * kSelThreads;
+#pragma unroll
+    for (int r = 0; r < kSelRows; ++r) d[r][0][e] = d[r][1][e] = j < n && j != i0 + r ? 0.0 : NAN;
+  }
+  // reference order of operations: columns in turn, each square rounded
+  auto distances = [&](const double* __restrict__ x, int p, int space) {
+    for (int c = 0; c < p; ++c) {
+      const double* const col = x + static_cast<long long>(c) * n;
+      double xi[kSelRows];
+#pragma unroll
+      for (int r = 0; r < kSelRows; ++r) xi[r] = col[min(i0 + r, n - 1)];
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int j = tid + e * kSelThreads;
+        const double xj = col[min(j, n - 1)];
+#pragma unroll
+        for (int r = 0; r < kSelRows; ++r) {
+          const double delta = __dsub_rn(xi[r], xj);
+          d[r][space][e] = __dadd_rn(d[r][space][e], __dmul_rn(delta, delta));
+        }
+      }
+    }
+  };
+  distances(high, p_high, 0);
+  distances(low, p_low, 1);
+
+  int turn = 0;
+  // sum over the workgroup of a per-wave count, in every thread
+  auto total = [&](int c) {
+    if (lane == 0) cnt[turn][wave] = c;
+    __syncthreads();
+    int s = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s += cnt[turn][w];
+    turn ^= 1;
+    return s;
+  };
+
+#pragma unroll
+  for (int r = 0; r < kSelRows; ++r) {
+    const int i = i0 + r;
+    if (i >= n) break;  // whole block
+    bool fits = true;
+#pragma unroll
+    for (int sp = 0; sp < 2; ++sp) {
+      // smallest and largest distance (NaN left out by fmin and fmax)
+      double lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        lo = fmin(lo, d[r][sp][e]);
+        hi = fmax(hi, d[r][sp][e]);
+      }
+      for (int off = 32; off > 0; off >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, off));
+        hi = fmax(hi, __shfl_xor(hi, off));
+      }
+      __syncthreads();  // red, row are free
+      if (lane == 0) {
+        red[sp][0][wave] = lo;
+        red[sp][1][wave] = hi;
+      }
+      if (tid < 2) row.count[tid] = 0;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        lo = fmin(lo, red[sp][0][w]);
+        hi = fmax(hi, red[sp][1][w]);
+      }
+      double t = hi;
+      bool found = false;
+      for (int step = 0; step < 48; ++step) {
+        int c = 0;
+#pragma unroll
+        for (int e = 0; e < PER; ++e) c += __popcll(__ballot(d[r][sp][e] <= t));
+        c = total(c);
+        if (c >= kmax && c <= kSelCand) {
+          found = true;
+          break;
+        }
+        if (c < kmax)
+          lo = t;
+        else
+          hi = t;
+        t = lo + 0.5 * (hi - lo);
+        if (!(t > lo && t < hi)) break;
+      }
+      fits = fits && found;
+      if (!found) continue;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        if (d[r][sp][e] <= t) {
+          const int at = atomicAdd(&row.count[sp], 1);
+          row.cand_d[sp][at] = d[r][sp][e];
+          row.cand_j[sp][at] = tid + e * kSelThreads;
+        }
+      }
+      __syncthreads();
+      const int c = row.count[sp];
+      if (tid < c) {
+        const double dm = row.cand_d[sp][tid];
+        const int jm = row.cand_j[sp][tid];
+        int before = 0;
+        for (int q = 0; q < c; ++q) {
+          const double dq = row.cand_d[sp][q];
+          before += dq < dm || (dq == dm && row.cand_j[sp][q] < jm) ? 1 : 0;
+        }
+        if (before < kmax) row.nb[sp][before] = jm;
+      }
+    }
+    if (!fits) {  // whole block
+      if (tid == 0) todo[1 + atomicAdd(todo, 1)] = i;
+      continue;
+    }
+    __syncthreads();
+    // the neighbours' distances in the other space, from the threads that
+    // hold them; ranks start at 1
+    for (int q = 0; q < 2 * kmax; ++q) {
+      const int sp = q >= kmax ? 1 : 0, at = q - sp * kmax;
+      const int j = row.nb[sp][at];
+      if ((j & (kSelThreads - 1)) == tid) {
+        double v = 0.0;
+#pragma unroll
+        for (int e = 0; e < PER; ++e)
+          if (e == j / kSelThreads) v = sp == 0 ? d[r][1][e] : d[r][0][e];
+        row.other[sp][at] = v;
+        row.rank[sp][at] = 1;
+      }
+    }
+    __syncthreads();
+    for (int sp = 0; sp < 2; ++sp) {
+      for (int at = 0; at < kmax; ++at) {
+        const double v = row.other[sp][at];
+        const int j = row.nb[sp][at];
+        int c = 0;
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+          const double w = sp == 0 ? d[r][1][e] : d[r][0][e];
+          c += __popcll(__ballot(w < v || (w == v && tid + e * kSelThreads < j)));
+        }
+        if (lane == 0 && c != 0) atomicAdd(&row.rank[sp][at], c);
+      }
+    }
+    __syncthreads();
+    // the sums of each requested k (integer-valued: exact in any order)
+    if (wave == 0) {
+      for (int q = 0; q < nk; ++q) {
+        const int k = ks[q];
+        double shared = 0.0, trust = 0.0, cont = 0.0, rerr = 0.0;
+        if (lane < k) {
+          const int in_high = row.rank[1][lane], in_low = row.rank[0][lane];
+          if (in_high <= k) shared = 1.0;
+          if (in_high > k) trust = in_high - k;
+          if (in_low > k) cont = in_low - k;
+          rerr = abs(in_high - (lane + 1));
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+          shared += __shfl_xor(shared, off);
+          trust += __shfl_xor(trust, off);
+          cont += __shfl_xor(cont, off);
+          rerr += __shfl_xor(rerr, off);
+        }
+        if (lane == 0) {
+          double* const out = sums + (static_cast<long long>(i) * nk + q) * 4;
+          out[0] = shared;
+          out[1] = trust;
+          out[2] = cont;
+          out[3] = rerr;
+        }
+      }
+    }
   }
 }
 
@@ -211,8 +439,28 @@ int structure_metrics_run(const double* high, int n, int p_high, const double* l
   if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_structure_rows),
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))) != hipSuccess)
     return fail("structure metrics LDS");
-  k_structure_rows<<<n, kMetThreads, lds, nullptr>>>(dh.p, p_high, dl.p, p_low, n, m, dks.p, nk, kmax, dsums.p);
-  if ((e = hipGetLastError()) != hipSuccess) return fail("structure metrics launch");
+  int sorted = n;  // rows for k_structure_rows
+  MetBuf<int> todo;  // their number, then the rows
+  if (kmax <= kSelMaxK && n >= kSelMinRows) {
+    if ((e = todo.alloc(static_cast<std::size_t>(n) + 1)) != hipSuccess ||
+        (e = hipMemset(todo.p, 0, sizeof(int))) != hipSuccess)
+      return fail("hipMalloc(structure metrics rows)");
+    const int blocks = (n + kSelRows - 1) / kSelRows;
+    if (n <= 4 * kSelThreads)
+      k_structure_select<4><<<blocks, kSelThreads, 0, nullptr>>>(dh.p, p_high, dl.p, p_low, n, dks.p, nk, kmax,
+                                                                 dsums.p, todo.p);
+    else
+      k_structure_select<10><<<blocks, kSelThreads, 0, nullptr>>>(dh.p, p_high, dl.p, p_low, n, dks.p, nk, kmax,
+                                                                  dsums.p, todo.p);
+    if ((e = hipGetLastError()) != hipSuccess) return fail("structure metrics launch");
+    if ((e = hipMemcpy(&sorted, todo.p, sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess)
+      return fail("hipMemcpy(structure metrics rows)");
+  }
+  if (sorted > 0) {
+    k_structure_rows<<<sorted, kMetThreads, lds, nullptr>>>(dh.p, p_high, dl.p, p_low, n, m, dks.p, nk, kmax,
+                                                            todo.p != nullptr ? todo.p + 1 : nullptr, dsums.p);
+    if ((e = hipGetLastError()) != hipSuccess) return fail("structure metrics launch");
+  }
   std::vector<double> sums(static_cast<std::size_t>(n) * nk * 4);
   if ((e = hipMemcpy(sums.data(), dsums.p, sums.size() * sizeof(double), hipMemcpyDeviceToHost)) != hipSuccess)
     return fail("hipMemcpy(structure metrics)");

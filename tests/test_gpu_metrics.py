@@ -50,6 +50,23 @@ def test_ties_and_identity(hip):
     np.testing.assert_array_equal(m[0], [1.0, 1.0, 1.0, 0.0])
 
 
+@pytest.mark.parametrize("n,ks", [(3, [1]), (97, [1, 64]), (1024, [5]), (1025, [1]), (1025, [64, 2]), (1535, [65]),
+                                  (1537, [15]), (2048, [15]), (2049, [64])])
+def test_selection_edges(hip, n, ks):
+    """Row counts at the edges of the selection's threads and registers, the
+    smallest and largest k that select and the first that sorts; a third of
+    the rows are copies of one row, more equal distances than the candidates
+    hold (those rows are sorted)."""
+    _say(f"case: structure metrics selection n={n} k={ks}")
+    rng = np.random.default_rng(n)
+    high = rng.normal(size=(n, 6))
+    high[rng.permutation(n)[:n // 3]] = high[0]
+    low = np.round(rng.normal(size=(n, 2)) * 4) / 4
+    np.testing.assert_array_equal(_gpu(high, low, ks), mo.exact_structure_metrics(high, low, ks))
+    far = high * 1e200  # squared distances overflow to infinity
+    np.testing.assert_array_equal(_gpu(far, low, ks), mo.exact_structure_metrics(far, low, ks))
+
+
 def test_errors(hip):
     _say("case: structure metrics errors")
     x = np.zeros((10, 2))
