@@ -17,6 +17,7 @@ from dataclasses import dataclass, field
 import numpy as np
 
 from . import _lib
+from .layout import column_major
 from .session import TsneSession
 
 OPTIMIZER_LABEL = "opentsne_fitsne_fft_grid_native_hip"
@@ -83,22 +84,34 @@ def strip_self_neighbors(indices: np.ndarray, distances: np.ndarray, float32: bo
     Returns (indices, distances, has_self).  A self entry is the row's own
     index at distance <= tolerance; when every row has one, it is removed.
     """
+    return _strip_self(indices, distances, float32)[:3]
+
+
+# Rows looked at first for a self entry: one row without any decides that none
+# is stripped, and the whole comparison (n x k, three passes) is left out.
+_SELF_PROBE_ROWS = 256
+
+
+def _strip_self(indices: np.ndarray, distances: np.ndarray, float32: bool):
+    """strip_self_neighbors, and the input's index offset (None for k = 0)."""
     n, k = indices.shape
     if k < 1:
-        return indices, distances, False
+        return indices, distances, False, None
+    offset = knn_index_offset(indices)
     tol = max(math.sqrt(np.finfo(np.float32).eps), 1e-6) if float32 else max(math.sqrt(np.finfo(np.float64).eps), 1e-12)
-    expected = np.arange(n) + knn_index_offset(indices)
+    expected = np.arange(n) + offset
     if np.all((indices[:, 0] == expected) & (distances[:, 0] <= tol)):
-        return indices[:, 1:], distances[:, 1:], True
-    mask = (indices == expected[:, None]) & (distances <= tol)
-    if not np.all(mask.any(axis=1)):
-        return indices, distances, False
+        return indices[:, 1:], distances[:, 1:], True, offset
+    for rows in (slice(0, _SELF_PROBE_ROWS), slice(0, n)):
+        mask = (indices[rows] == expected[rows, None]) & (distances[rows] <= tol)
+        if not np.all(mask.any(axis=1)):
+            return indices, distances, False, offset
     if k == 1:
-        return indices[:, :0], distances[:, :0], True
+        return indices[:, :0], distances[:, :0], True, offset
     first = mask.argmax(axis=1)
     keep = np.ones((n, k), bool)
     keep[np.arange(n), first] = False
-    return indices[keep].reshape(n, k - 1), distances[keep].reshape(n, k - 1), True
+    return indices[keep].reshape(n, k - 1), distances[keep].reshape(n, k - 1), True, offset
 
 
 def normalize_negative_gradient_method(method: str) -> str:
@@ -210,7 +223,7 @@ def opentsne_knn(indices, distances=None, n_neighbors: int | None = None, perple
     else:
         idx0, dist0 = _coerce_knn(indices, distances)
         float32_input = dist0.dtype == np.float32
-        idx_s, dist_s, has_self = strip_self_neighbors(idx0, dist0, float32=float32_input)
+        idx_s, dist_s, has_self, offset = _strip_self(idx0, dist0, float32_input)
         n = idx_s.shape[0]
         available = idx_s.shape[1]
     if available < 1:
@@ -282,8 +295,9 @@ def opentsne_knn(indices, distances=None, n_neighbors: int | None = None, perple
             raise ValueError("incorrect format for `Y_init`.")
 
     if device_knn is None:
-        offset = knn_index_offset(idx_m)
-        idx_c = np.asfortranarray(idx_m, dtype=np.int32)
+        if has_self or k < available:  # other entries than the offset was found from
+            offset = knn_index_offset(idx_m)
+        idx_c = column_major(idx_m, np.int32)
     else:
         # column-major n x k: the first n_neighbors columns are a prefix of the buffers
         offset = int(getattr(device_knn, "index_base", 1))
@@ -297,7 +311,7 @@ def opentsne_knn(indices, distances=None, n_neighbors: int | None = None, perple
         # Session route: same kernels, with the exact KL every 50 iterations
         # when costs are recorded, and the interpolation grid when asked for.
         if device_knn is None:
-            sess = TsneSession(idx_c, np.asfortranarray(dist_m, dtype=np.float32), perplexity=perplexity,
+            sess = TsneSession(idx_c, column_major(dist_m, np.float32), perplexity=perplexity,
                                index_offset=offset)
         else:
             sess = TsneSession(perplexity=perplexity, index_offset=offset, n=n, k=k,
@@ -344,11 +358,11 @@ def opentsne_knn(indices, distances=None, n_neighbors: int | None = None, perple
             idx_p, dist_p = C.c_void_p(device_knn.indices_ptr), C.c_void_p(device_knn.distances_ptr)
             fn = lib.fastembedr_hip_opentsne_fft_from_device_knn_float
         elif dist_m.dtype == np.float64:
-            dist_c = np.asfortranarray(dist_m, dtype=np.float64)
+            dist_c = column_major(dist_m, np.float64)
             idx_p, dist_p = C.c_void_p(idx_c.ctypes.data), C.c_void_p(dist_c.ctypes.data)
             fn = lib.fastembedr_hip_opentsne_fft_from_knn
         else:
-            dist_c = np.asfortranarray(dist_m, dtype=np.float32)
+            dist_c = column_major(dist_m, np.float32)
             idx_p, dist_p = C.c_void_p(idx_c.ctypes.data), C.c_void_p(dist_c.ctypes.data)
             fn = lib.fastembedr_hip_opentsne_fft_from_knn_float
         init_p = None if init is None else C.c_void_p(init.ctypes.data)

@@ -11,6 +11,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
+from .layout import column_major
 
 
 def _ptr(a: np.ndarray | None) -> C.c_void_p | None:
@@ -39,8 +40,8 @@ class TsneSession:
             on_device = 1
             self.n, self.k = int(n), int(k)
         else:
-            idx = np.asfortranarray(indices, dtype=np.int32)
-            dist = np.asfortranarray(distances, dtype=np.float32)
+            idx = column_major(indices, np.int32)
+            dist = column_major(distances, np.float32)
             if idx.shape != dist.shape or idx.ndim != 2:
                 raise ValueError("KNN `indices` and `distances` must have the same dimensions.")
             self.n, self.k = idx.shape

@@ -19,6 +19,7 @@ from dataclasses import dataclass, field
 import numpy as np
 
 from . import _lib
+from .layout import column_major
 
 INITIALIZATIONS = {"median": 0, "weighted": 1, "random": 2}
 NA_SEED = -(2 ** 31)  # R's NA_integer_
@@ -55,7 +56,7 @@ def _coerce_query_knn(knn, n_reference: int, k: int | None):
         if k > idx.shape[1]:
             raise ValueError("`k` cannot be larger than the available reference count.")
         idx, dist = idx[:, :k], dist[:, :k]
-    return np.asfortranarray(idx, dtype=np.int32), np.asfortranarray(dist)
+    return column_major(idx, np.int32), column_major(dist, np.float64)
 
 
 def transform_tsne(reference_layout, knn=None, reference_data=None, new_data=None, k: int | None = None,

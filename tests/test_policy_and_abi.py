@@ -73,6 +73,46 @@ def test_strip_self_neighbors():
     assert not has4 and i4.shape == (n, k - 1)
 
 
+@pytest.mark.parametrize("bad_row", [None, 0, 255, 256, 699])
+def test_strip_self_neighbors_probe(bad_row):
+    """Self entries off the first column, and one row without any before, at
+    and past the rows that are looked at first."""
+    rng = np.random.default_rng(5)
+    n, k = 700, 6
+    idx = np.stack([rng.permutation(n)[:k] for _ in range(n)]).astype(np.int32)
+    idx[idx == np.arange(n)[:, None]] = 0
+    dist = np.sort(rng.uniform(0.5, 1.0, (n, k)).astype(np.float32), axis=1)
+    at = rng.integers(1, k, n)
+    idx[np.arange(n), at] = np.arange(n)
+    dist[np.arange(n), at] = 0.0
+    if bad_row is not None:
+        dist[bad_row, at[bad_row]] = 0.25
+    i2, d2, has = opentsne.strip_self_neighbors(idx, dist)
+    assert has == (bad_row is None)
+    if has:
+        keep = np.arange(k)[None, :] != at[:, None]
+        np.testing.assert_array_equal(i2, idx[keep].reshape(n, k - 1))
+        np.testing.assert_array_equal(d2, dist[keep].reshape(n, k - 1))
+    else:
+        assert i2 is idx and d2 is dist
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 3000])
+def test_column_major_copies(n):
+    from fastembedr_amd.layout import column_major
+
+    base = np.random.default_rng(n).integers(-5, 10 ** 6, (n, 9))
+    wide = np.arange(4 * n * 9).reshape(n, 36)
+    for a in (base, np.asfortranarray(base), base[:, :4], base[::-1], base[:, ::-1], wide[:, ::4], base.T.copy().T,
+              base[::2]):
+        for dtype in (np.int32, np.float32, np.float64, np.int64):
+            got = column_major(a, dtype)
+            assert got.dtype == dtype and got.flags.f_contiguous
+            np.testing.assert_array_equal(got, np.asfortranarray(a, dtype=dtype))
+    f = np.asfortranarray(base.astype(np.float32))
+    assert column_major(f, np.float32) is f
+
+
 def test_index_offset():
     assert opentsne.knn_index_offset(np.array([[1, 2], [2, 1]])) == 1
     assert opentsne.knn_index_offset(np.array([[0, 1], [1, 0]])) == 0
