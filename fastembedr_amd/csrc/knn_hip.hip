@@ -24,12 +24,12 @@
 //     4m + 2h and 4m + 2h + 1 for half h, so both halves of the wave cover
 //     the four dimensions of chunk m).  Per (query, reference) the scan
 //     keeps s = |r|^2 - 2 q.r, which orders references as |q - r|^2 does.
-//     Each query keeps a threshold t (the kp-th smallest s seen, +inf until
-//     kp were seen) and a candidate buffer of B entries in global memory;
-//     slots come from ballots (a wave owns its rows), and when a buffer
-//     could overflow in the next tile the wave sorts it (bitonic across its
-//     64 lanes) and keeps the kp best.  The host picks B >= 2 kp + 64, so
-//     compactions are rare once t has settled.
+//     Each query keeps a threshold t (at or above the kp-th smallest s seen;
+//     +inf until kp were seen) and a candidate buffer of B entries in global
+//     memory; slots come from ballots (a wave owns its rows), and a buffer
+//     that could overflow in the next tile is cut to kp (and up to kKnnSlack
+//     more) at a value found by bisection.  B has room for three kp, so cuts
+//     are rare once t has settled.
 //  3. finalize (k_knn_finalize): per query, the candidates' squared
 //     distances are recomputed from the input rows in fp64, the query itself
 //     is dropped on request, and the rest are sorted by (d2, index); the
