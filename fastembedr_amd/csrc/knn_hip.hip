@@ -1620,9 +1620,14 @@ hipError_t knn_projection_basis(const float* x, Strides st, int n, int d, const 
   k_knn_cov_sum<<<dim3(col_blocks, d), 256, 0, stream>>>(cov, d, parts);
   k_knn_proj_random<<<value_blocks, 256, 0, stream>>>(q_dev, values);
   for (int it = 0; it < kProjIters; ++it) {
+    // the second Gram-Schmidt round only where Q is handed on: the iterations
+    // before it need the columns' span and scale, not their last digits
+    // (20,000 x 784 cosine, k = 30, whole call 19.1 ms with two rounds
+    // throughout, 17.6 so)
+    const int rounds = it + 1 < kProjIters ? 1 : 2;
     k_knn_cov_times<<<(d + 3) / 4, kProjDim, 0, stream>>>(cov, q_dev, d, y_dev);
     for (int p0 = 0; p0 < kProjDim; p0 += kProjPanel) {
-      for (int round = 0; round < 2; ++round) {
+      for (int round = 0; round < rounds; ++round) {
         const int blocks = p0 + (round == 0 ? kProjPanel : 0);
         if (blocks > 0) k_knn_proj_coef<<<blocks, 256, 0, stream>>>(y_dev, d, p0, coef, norms);
         if (p0 > 0) k_knn_proj_update<<<dim3(col_blocks, kProjPanel), 256, 0, stream>>>(y_dev, d, p0, coef);
